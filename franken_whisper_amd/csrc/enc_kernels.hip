@@ -530,90 +530,110 @@ __global__ void k_fill_u16(uint16_t *p, size_t n, uint16_t v) {
 
 // ---------------------------------------------------------------------------
 // Attention on f16 pairs (S^T = K Q^T, online softmax over 64-key tiles,
-// O^T += V^T P^T), with 8 waves (256 queries) per block sharing each K/V tile, and the tiles (K hi/lo, V^T hi/lo:
-// 4 x 8 KB) fed global -> LDS directly through an AT_NS-stage ring, one
-// barrier per tile.  Rows are 128 bytes; 16-byte chunk c of row r sits at
-// chunk c ^ (r & 7), which keeps the fragment reads free of bank conflicts.
-// QPW 32-query sub-tiles per wave share each K / V^T fragment read from LDS
-// (the fragment reads, not the MFMAs, set the LDS traffic per query), every
-// query's arithmetic the same whatever QPW is.  Measured on MI355X (16
-// large-v3-turbo windows, per launch): 8 waves x 2 sub-tiles with a 2-stage
-// ring 550 us; 8 x 1 with 3 stages 620 us; 8 x 1 with 2 stages 608 us;
-// 4 x 2 with 2 stages 601 us; 4 x 2 with 3 stages 724 us.
-#ifndef AT_QW
-#define AT_QW 8
-#endif
-#ifndef AT_NSTAGE
-#define AT_NSTAGE 2
-#endif
-#ifndef AT_QPW
-#define AT_QPW 2
-#endif
-template <int AT_QW_, int AT_NS, int QPW>
-__global__ void __launch_bounds__(64 * AT_QW_, 2) k_attention2(const uint16_t *qh, const uint16_t *ql, const uint16_t *kh,
-                                                           const uint16_t *kl, const uint16_t *vth, const uint16_t *vtl,
-                                                           int T, int Tp, int H, int d, int out_mode, float *of,
-                                                           uint16_t *oh, uint16_t *ol) {
-    __shared__ __align__(1024) uint16_t sm[AT_NS][4][64 * 64]; // [stage][K hi, K lo, V^T hi, V^T lo][row][64]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int h = blockIdx.y, b = blockIdx.z;
-    const size_t bh = (size_t)b * H + h;
-    const int q0 = (blockIdx.x * AT_QW_ + wave) * 32 * QPW;
+// O^T += V^T P^T).
+//
+// The MFMAs (three f16 products per f32 product) and the softmax's VALU work
+// take about the same time, so they have to run side by side.  A block is two
+// groups of 4 waves, one wave of each group per SIMD, and group 1 runs one
+// phase behind: while one group multiplies (P V of its last tile, then the
+// scores of its next) the other one exponentiates.  A barrier ends each phase.
+//
+// The tiles (K hi/lo, V^T hi/lo: 4 x 8 KB) go global -> LDS through a ring of
+// two slots shared by both groups; slot j % 2 holds the K of tile j and the V of
+// tile j - 1, which one multiply phase uses together.  Rows are 128 bytes;
+// 16-byte chunk c of row r sits at chunk c ^ (r & 7), which keeps the fragment
+// reads free of bank conflicts.  QPW 32-query sub-tiles per wave share each
+// K / V^T fragment read; every query's arithmetic is the same whatever QPW is.
+//
+// What bounds it: per 64-key tile a wave of QPW 2 issues 96 MFMAs (33 cycles
+// each) and about as many cycles of VALU work; a tile pair takes 8,000 cycles
+// (13,000 when every wave did both in step), and the clock falls to ~1.4 GHz
+// under that load, so the matrix units' power is what is left.  Measured, 1,500
+// rows of 20 heads: 10 windows 416 -> 350 us a launch, 16 windows 610 -> 520;
+// one window (120 blocks, half the CUs) 59 -> 57.
+#define AT_TILE (64 * 64) // halves of one array's tile
+// The f16 pairs of four values: hi = f16(v), lo = f16(v - hi), one mixed-precision
+// fma per lo (v - hi is exact, then rounded once).  One asm block, so that a low
+// half's write is never followed at once by the write of its register's high half.
+__device__ __forceinline__ void at_split4(const float (&v)[4], uint32_t &h0, uint32_t &h1, uint32_t &l0,
+                                          uint32_t &l1) {
+    const v2f a = {v[0], v[1]}, c = {v[2], v[3]};
+    h0 = __builtin_bit_cast(uint32_t, __builtin_convertvector(a, v2h));
+    h1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(c, v2h));
+    asm("v_fma_mixlo_f16 %0, %2, 1.0, -%6 op_sel:[0,0,0] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %1, %4, 1.0, -%7 op_sel:[0,0,0] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %0, %3, 1.0, -%6 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %1, %5, 1.0, -%7 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+        : "=&v"(l0), "=&v"(l1)
+        : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(h0), "v"(h1));
+}
+// the maximum / sum of lanes i and i ^ 32
+__device__ __forceinline__ float at_max32(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float at_sum32(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+template <int QPW>
+__global__ void __launch_bounds__(512, 2) k_attention3(const uint16_t *qh, const uint16_t *ql, const uint16_t *kh,
+                                                       const uint16_t *kl, const uint16_t *vth, const uint16_t *vtl,
+                                                       int T, int Tp, int H, int d, int nq, int out_mode, float *of,
+                                                       uint16_t *oh, uint16_t *ol) {
+    __shared__ __align__(1024) uint16_t sm[2][4][AT_TILE]; // [slot][K hi, K lo, V^T hi, V^T lo][row][64]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int grp = wave >> 2;
+    // Blocks are dealt round-robin to the 8 XCDs: give each XCD a contiguous
+    // run of (window, head, query block), so a head's K / V stay in one L2
+    const int nb = gridDim.x, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3, per = nb >> 3, rem = nb & 7;
+    const int bt = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
+    const size_t bh = bt / nq;
+    const int b = (int)(bh / H), h = (int)(bh - (size_t)b * H);
+    const int q0 = ((bt - (int)bh * nq) * 8 + wave) * 32 * QPW;
     const int nt = (T + 63) >> 6;
     // this lane's Q^T fragments: q = q0 + 32 qs + l % 32, dims ks*16 + (l/32)*8 .. +8
     v8h qfh[QPW][4], qfl[QPW][4];
 #pragma unroll
     for (int qs = 0; qs < QPW; qs++) {
         const int myq = q0 + qs * 32 + (lane & 31);
-        const int qc = myq < T ? myq : T - 1;
+        const int qc = myq < T ? myq : T - 1; // queries past T repeat the last one and are not stored
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
             const int dd = ks * 16 + (lane >> 5) * 8;
-            v8h a = *(const v8h *)(qh + (bh * T + qc) * 64 + dd), c = *(const v8h *)(ql + (bh * T + qc) * 64 + dd);
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                qfh[qs][ks][e] = myq < T ? a[e] : (_Float16)0.0f;
-                qfl[qs][ks][e] = myq < T ? c[e] : (_Float16)0.0f;
-            }
+            qfh[qs][ks] = *(const v8h *)(qh + (bh * T + qc) * 64 + dd);
+            qfl[qs][ks] = *(const v8h *)(ql + (bh * T + qc) * 64 + dd);
         }
     }
-    // loader: 32 instructions of 1 KB per tile, AT_QW_ waves share them
-    constexpr int LPW = 32 / AT_QW_;
-    const uint16_t *src[LPW];
-    int dsto[LPW];
-#pragma unroll
-    for (int qq = 0; qq < LPW; qq++) {
-        const int ii = wave * LPW + qq, arr = ii >> 3, r = ((ii & 7) << 3) + (lane >> 3);
-        const int c = (lane & 7) ^ (r & 7);
-        dsto[qq] = arr * 64 * 64 + ((ii & 7) << 3) * 64; // halves, wave-uniform
-        if (arr < 2) src[qq] = (arr ? kl : kh) + (bh * T) * 64 + (size_t)r * 64 + c * 8;  // + key0*64 per tile
-        else src[qq] = (arr == 3 ? vtl : vth) + (bh * 64 + r) * (size_t)Tp + c * 8;       // + key0 per tile
-    }
-    auto issue = [&](int it) {
-        const int itc = it < nt ? it : nt - 1;
-        const int k0 = itc * 64;
-        uint16_t *base = &sm[it % AT_NS][0][0];
-#pragma unroll
-        for (int qq = 0; qq < LPW; qq++) {
-            const int ii = wave * LPW + qq, arr = ii >> 3;
-            const uint16_t *g;
-            if (arr < 2) {
-                // key rows past T reload row T-1 (masked in the softmax)
-                const int r = ((ii & 7) << 3) + (lane >> 3);
-                const int kr = k0 + r < T ? k0 : T - 1 - r;
-                g = src[qq] + (size_t)kr * 64;
-            } else {
-                g = src[qq] + k0; // V^T rows are zero padded to Tp >= 64 * nt
-            }
-            __builtin_amdgcn_global_load_lds((const void *)g,
-                                             (void __attribute__((address_space(3))) *)(base + dsto[qq]), 16, 0, 0);
+    // loader: half of array wave / 2 of the pair, 4 instructions of 8 rows (1 KB)
+    // each (uniform base + 32-bit lane offset: no address registers per row group)
+    const int arr = wave >> 1, r0 = (wave & 1) * 32, lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
+    const uint32_t lstep = arr < 2 ? 64 : Tp; // row stride in halves
+    const uint32_t loff = (lr * lstep + lc) * 2;
+    const char *src = (const char *)((arr == 0 ? kh + bh * T * 64 : arr == 1 ? kl + bh * T * 64
+                                      : arr == 2 ? vth + bh * 64 * Tp : vtl + bh * 64 * Tp) + (size_t)r0 * lstep);
+    auto issue = [&](int j) {
+        if (arr < 2 ? j >= nt : (j == 0 || j > nt)) return;
+        const int k0 = (j - (arr < 2 ? 0 : 1)) * 64;
+        uint16_t *base = &sm[j & 1][arr][r0 * 64];
+        if (arr < 2 && k0 + 64 > T) {
+            // the last tile's key rows past T reload row T - 1 (masked in the softmax)
+#pragma unroll 1
+            for (int q = 0; q < 4; q++)
+                __builtin_amdgcn_global_load_lds(
+                    (const void *)(src + ((min(k0 + r0 + q * 8 + lr, T - 1) - r0) * 64 + lc) * 2),
+                    (void __attribute__((address_space(3))) *)(base + q * 512), 16, 0, 0);
+            return;
         }
+        // (V^T rows are zero padded to Tp >= 64 * nt)
+        const char *p = src + (size_t)(arr < 2 ? k0 * 64 : k0) * 2;
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            __builtin_amdgcn_global_load_lds((const void *)(p + (size_t)(q * 16 * lstep) + loff),
+                                             (void __attribute__((address_space(3))) *)(base + q * 512), 16, 0, 0);
     };
-    // Each accumulator takes all three f16-pair products in turn (hi*hi,
-    // lo*hi, hi*lo); the two 32-key (or 32-dim) halves and the sub-tiles are
-    // independent chains, interleaved so consecutive MFMAs never depend on
-    // each other.
-    v16f o[QPW][2];
+    v16f o[QPW][2], st[QPW][2];
+    uint32_t ph[QPW][2][8], pl[QPW][2][8];
     float m[QPW], l[QPW];
 #pragma unroll
     for (int qs = 0; qs < QPW; qs++) {
@@ -625,45 +645,74 @@ __global__ void __launch_bounds__(64 * AT_QW_, 2) k_attention2(const uint16_t *q
             for (int r = 0; r < 16; r++) o[qs][j][r] = 0.0f;
     }
     const float sl2 = 0.125f * 1.4426950408889634f;
+    // The four fragments of step s of an array pair: rows l % 32 of both
+    // 32-row halves, chunk 2 s + l / 32, hi then lo.
+    const int fr = lane & 31, fx = lane & 7, fh = lane >> 5;
+    auto frag = [&](const uint16_t *a, int s, v8h (&f)[4]) {
+        const int off = fr * 64 + (((s * 2 + fh) ^ fx) << 3);
+        f[0] = *(const v8h *)(a + off);
+        f[1] = *(const v8h *)(a + 32 * 64 + off);
+        f[2] = *(const v8h *)(a + AT_TILE + off);
+        f[3] = *(const v8h *)(a + AT_TILE + 32 * 64 + off);
+    };
+    // Each accumulator takes all three products in turn (hi*hi, lo*hi, hi*lo);
+    // the two 32-row halves and the sub-tiles are independent chains,
+    // interleaved so consecutive MFMAs never depend on each other.  The next
+    // step's fragments are read under the current step's MFMAs.
+    auto mfma12 = [&](const v8h (&f)[4], auto &acc, auto bhi, auto blo) {
 #pragma unroll
-    for (int p = 0; p < AT_NS - 1; p++) issue(p);
-    for (int it = 0; it < nt; it++) {
-        FW_WAIT_VM_LGKM0(LPW * (AT_NS - 2)); // this wave's loads of tile `it` have landed
-        asm volatile("s_barrier" ::: "memory");
-        issue(it + AT_NS - 1);
-        const uint16_t *sK = &sm[it % AT_NS][0][0];
-        const int k0 = it * 64;
-        // the first MFMA of each chain takes a zero accumulator operand
-        const v16f zero = {};
-        v16f st[QPW][2];
+        for (int qs = 0; qs < QPW; qs++)
 #pragma unroll
-        for (int qs = 0; qs < QPW; qs++) st[qs][0] = st[qs][1] = zero;
+            for (int t = 0; t < 2; t++)
+                acc[qs][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[t], bhi(qs), acc[qs][t], 0, 0, 0);
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-            v8h ah[2], al[2];
+        for (int qs = 0; qs < QPW; qs++)
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const int kr = t * 32 + (lane & 31), c = ks * 2 + (lane >> 5);
-                const int off = kr * 64 + ((c ^ (kr & 7)) << 3);
-                ah[t] = *(const v8h *)(sK + off);
-                al[t] = *(const v8h *)(sK + 64 * 64 + off);
+            for (int t = 0; t < 2; t++)
+                acc[qs][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[2 + t], bhi(qs), acc[qs][t], 0, 0, 0);
+#pragma unroll
+        for (int qs = 0; qs < QPW; qs++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+                acc[qs][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[t], blo(qs), acc[qs][t], 0, 0, 0);
+    };
+    // The multiply phase on slot j % 2: with V, O += V P of tile j - 1; with K,
+    // the scores of tile j.  Steps 0-3 are V's 16-key groups, 4-7 K's 16 dims.
+    // P holds keys {G + 4h + 0..3, G + 8 + 4h + 0..3} (G = 16 s, h = lane / 32);
+    // V^T stores each 16-key group with bits 2 and 3 of the key swapped, so
+    // these 8 keys are one 16-byte chunk.
+    auto mult = [&](int j, auto hasv, auto hask) {
+        constexpr int S0 = decltype(hasv)::value ? 0 : 4, S1 = decltype(hask)::value ? 8 : 4;
+        const uint16_t *sl = &sm[j & 1][0][0];
+        v8h f[2][4];
+        auto rd = [&](int s) { frag(sl + (s < 4 ? 2 * AT_TILE : 0), s & 3, f[s & 1]); };
+        rd(S0);
+#pragma unroll
+        for (int s = S0; s < S1; s++) {
+            // the step's fragments were requested a whole step ago; waiting here
+            // keeps the next step's in flight under this step's MFMAs
+            FW_WAIT_LGKM0();
+            if (s + 1 < S1) rd(s + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (s < 4) {
+                auto pick = [&](const uint32_t (&p)[QPW][2][8], int qs) {
+                    const uint32_t *e = &p[qs][s >> 1][(s & 1) * 4];
+                    return __builtin_bit_cast(v8h, make_uint4(e[0], e[1], e[2], e[3]));
+                };
+                mfma12(f[s & 1], o, [&](int qs) { return pick(ph, qs); }, [&](int qs) { return pick(pl, qs); });
+            } else {
+                if (s == 4) {
+                    const v16f zero = {};
+#pragma unroll
+                    for (int qs = 0; qs < QPW; qs++) st[qs][0] = st[qs][1] = zero;
+                }
+                mfma12(f[s & 1], st, [&](int qs) { return qfh[qs][s - 4]; }, [&](int qs) { return qfl[qs][s - 4]; });
             }
-#pragma unroll
-            for (int qs = 0; qs < QPW; qs++) {
-                st[qs][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[0], qfh[qs][ks], st[qs][0], 0, 0, 0);
-                st[qs][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[1], qfh[qs][ks], st[qs][1], 0, 0, 0);
-            }
-#pragma unroll
-            for (int qs = 0; qs < QPW; qs++) {
-                st[qs][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[0], qfh[qs][ks], st[qs][0], 0, 0, 0);
-                st[qs][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[1], qfh[qs][ks], st[qs][1], 0, 0, 0);
-            }
-#pragma unroll
-            for (int qs = 0; qs < QPW; qs++) {
-                st[qs][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[0], qfl[qs][ks], st[qs][0], 0, 0, 0);
-                st[qs][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[1], qfl[qs][ks], st[qs][1], 0, 0, 0);
-            }
+            __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    auto softmax = [&](int j) {
+        const int k0 = j * 64;
         // keys past T exist only in the last tile
         if (k0 + 64 > T) {
 #pragma unroll
@@ -676,6 +725,9 @@ __global__ void __launch_bounds__(64 * AT_QW_, 2) k_attention2(const uint16_t *q
                         if (key >= T) st[qs][t][r] = -INFINITY;
                     }
         }
+        // the sub-tiles side by side: their chains (maximum, sum) are independent
+        float mnew[QPW], nms[QPW], psum[QPW];
+        bool moved = false;
 #pragma unroll
         for (int qs = 0; qs < QPW; qs++) {
             float tmax = -INFINITY;
@@ -683,88 +735,108 @@ __global__ void __launch_bounds__(64 * AT_QW_, 2) k_attention2(const uint16_t *q
             for (int t = 0; t < 2; t++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) tmax = fmaxf(tmax, st[qs][t][r]);
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-            const float mnew = fmaxf(m[qs], tmax);
+            mnew[qs] = fmaxf(m[qs], at_max32(tmax));
             // exp2((s - mnew) * sl2) as one fma per score
-            const float nms = -mnew * sl2;
-            float psum = 0.0f;
+            nms[qs] = -mnew[qs] * sl2;
+            psum[qs] = 0.0f;
+            moved |= mnew[qs] != m[qs];
+        }
+        // rescale only when some row's running max moved (wave-uniform test;
+        // alpha is exactly 1 where it did not)
+        if (__builtin_amdgcn_ballot_w64(moved)) {
 #pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(st[qs][t][r], sl2, nms));
-                    st[qs][t][r] = pv;
-                    psum += pv;
-                }
-            psum += __shfl_xor(psum, 32, 64);
-            // rescale only when some row's running max moved (wave-uniform test)
-            if (__builtin_amdgcn_ballot_w64(mnew != m[qs])) {
-                const float alpha = __builtin_amdgcn_exp2f((m[qs] - mnew) * sl2);
+            for (int qs = 0; qs < QPW; qs++) {
+                const float alpha = __builtin_amdgcn_exp2f((m[qs] - mnew[qs]) * sl2);
                 l[qs] *= alpha;
 #pragma unroll
-                for (int j = 0; j < 2; j++)
+                for (int t = 0; t < 2; t++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) o[qs][j][r] *= alpha;
+                    for (int r = 0; r < 16; r++) o[qs][t][r] *= alpha;
             }
-            l[qs] += psum;
-            m[qs] = mnew;
         }
-        const uint16_t *sV = &sm[it % AT_NS][2][0];
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                // P holds keys {G + 4h + 0..3, G + 8 + 4h + 0..3} (G = 32t + 16u,
-                // h = lane / 32); V^T stores each 16-key group with bits 2 and 3
-                // of the key swapped, so these 8 keys are one 16-byte chunk
-                const int c = t * 4 + u * 2 + (lane >> 5);
-                v8h vh[2], vl[2];
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const int dim = j * 32 + (lane & 31);
-                    const int a = dim * 64 + ((c ^ (dim & 7)) << 3);
-                    vh[j] = *(const v8h *)(sV + a);
-                    vl[j] = *(const v8h *)(sV + 64 * 64 + a);
-                }
+            for (int r = 0; r < 16; r += 4)
 #pragma unroll
                 for (int qs = 0; qs < QPW; qs++) {
-                    // f16 pair of P, two values per conversion
-                    v8h ph, pl;
+                    float e[4];
 #pragma unroll
-                    for (int e = 0; e < 8; e += 2) {
-                        const v2f pv = {st[qs][t][8 * u + e], st[qs][t][8 * u + e + 1]};
-                        const v2h hh = __builtin_convertvector(pv, v2h);
-                        const v2h lo = __builtin_convertvector(pv - __builtin_convertvector(hh, v2f), v2h);
-                        ph[e] = hh[0];
-                        ph[e + 1] = hh[1];
-                        pl[e] = lo[0];
-                        pl[e + 1] = lo[1];
+                    for (int u = 0; u < 4; u++) {
+                        e[u] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[qs][t][r + u], sl2, nms[qs]));
+                        psum[qs] += e[u];
                     }
-                    o[qs][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[0], ph, o[qs][0], 0, 0, 0);
-                    o[qs][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[1], ph, o[qs][1], 0, 0, 0);
-                    o[qs][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[0], ph, o[qs][0], 0, 0, 0);
-                    o[qs][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl[1], ph, o[qs][1], 0, 0, 0);
-                    o[qs][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[0], pl, o[qs][0], 0, 0, 0);
-                    o[qs][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[1], pl, o[qs][1], 0, 0, 0);
+                    at_split4(e, ph[qs][t][r >> 1], ph[qs][t][(r >> 1) + 1], pl[qs][t][r >> 1], pl[qs][t][(r >> 1) + 1]);
                 }
-            }
+#pragma unroll
+        for (int qs = 0; qs < QPW; qs++) {
+            l[qs] += at_sum32(psum[qs]);
+            m[qs] = mnew[qs];
+        }
+    };
+    // every LDS access of the phase has completed before the barrier lets
+    // another wave refill what it read
+    auto phase_end = [&]() {
+        FW_WAIT_LGKM0();
+        asm volatile("s_barrier" ::: "memory");
+    };
+    // Phase 2j: group 0 multiplies pair j, group 1 exponentiates tile j - 1;
+    // phase 2j + 1: group 1 multiplies pair j, group 0 exponentiates tile j.
+    // Pair j + 2 is requested in phase 2j + 2, when nobody reads its slot any
+    // more, and waited for at the end of phase 2j + 3.
+    const std::true_type yes;
+    const std::false_type no;
+    issue(0);
+    FW_WAIT_VM(0);
+    phase_end();
+    issue(1);
+    if (grp) phase_end();
+    mult(0, no, yes);
+    if (grp) FW_WAIT_VM(0);
+    phase_end();
+    for (int j = 0; j + 1 < nt; j++) {
+        if (grp) issue(j + 2);
+        softmax(j);
+        if (!grp) FW_WAIT_VM(0);
+        phase_end();
+        if (!grp) issue(j + 2);
+        mult(j + 1, yes, yes);
+        if (grp) FW_WAIT_VM(0);
+        phase_end();
     }
-    FW_WAIT_VM(0); // dummy tiles landed before the block exits
+    softmax(nt - 1);
+    if (!grp) FW_WAIT_VM(0);
+    phase_end();
+    mult(nt, yes, no);
+    if (!grp) phase_end(); // group 1 started one barrier later
 #pragma unroll
     for (int qs = 0; qs < QPW; qs++) {
         const int myq = q0 + qs * 32 + (lane & 31);
         if (myq >= T) continue;
         const float inv = 1.0f / l[qs];
         const size_t orow = ((size_t)b * T + myq) * d + (size_t)h * 64;
+        // dims t*32 + q*8 + (lane/32)*4 .. +3 of the row
+        if (out_mode == 0) {
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+            for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int dim = j * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                const float v = o[qs][j][r] * inv;
-                if (out_mode == 0) of[orow + dim] = v;
-                else fw_split(v, oh[orow + dim], ol[orow + dim]);
-            }
+                for (int q = 0; q < 4; q++)
+                    *(float4 *)(of + orow + t * 32 + q * 8 + (lane >> 5) * 4) =
+                        make_float4(o[qs][t][q * 4] * inv, o[qs][t][q * 4 + 1] * inv, o[qs][t][q * 4 + 2] * inv,
+                                    o[qs][t][q * 4 + 3] * inv);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    uint16_t hi[4], lw[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) fw_split(o[qs][t][q * 4 + e] * inv, hi[e], lw[e]);
+                    const size_t oo = orow + t * 32 + q * 8 + (lane >> 5) * 4;
+                    *(uint2 *)(oh + oo) = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
+                    *(uint2 *)(ol + oo) = make_uint2(lw[0] | ((uint32_t)lw[1] << 16), lw[2] | ((uint32_t)lw[3] << 16));
+                }
+        }
     }
 }
 
@@ -1121,9 +1193,11 @@ void fw_launch_fill_u16(hipStream_t st, uint16_t *p, size_t n, uint16_t v) {
 void fw_launch_attention(hipStream_t st, const uint16_t *qh, const uint16_t *ql, const uint16_t *kh,
                          const uint16_t *kl, const uint16_t *vth, const uint16_t *vtl, int B, int T, int Tp, int H,
                          int d, int out_mode, float *of, uint16_t *oh, uint16_t *ol) {
-    // the largest query tile whose launch still covers every CU (one window:
-    // 20 heads x 12 blocks of 128 queries; ten: 20 x 10 x 3 of 512); every
-    // tile gives the same bits
+    // Rounds of the CUs (one block each) times the work of a block, which grows
+    // with QPW: 256 or 512 queries per block, the larger one where the smaller
+    // gains nothing (it reads the fragments once per two sub-tiles: 16 windows
+    // 490 us against 537; 10 windows, 3 rounds against 5 half ones, 351 against
+    // 342; two windows 108 against 75).
     static int n_cu = 0;
     if (!n_cu) {
         int dev = 0;
@@ -1131,12 +1205,12 @@ void fw_launch_attention(hipStream_t st, const uint16_t *qh, const uint16_t *ql,
         if (hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n_cu <= 0)
             n_cu = 256;
     }
-    auto nblk = [&](int qb) { return (long long)B * H * ((T + qb - 1) / qb); };
-#define AT_GO(QW_, QPW_)                                                                                           \
-    hipLaunchKernelGGL((k_attention2<QW_, AT_NSTAGE, QPW_>), dim3((T + 32 * QW_ * QPW_ - 1) / (32 * QW_ * QPW_), H, B), \
-                       dim3(64 * QW_), 0, st, qh, ql, kh, kl, vth, vtl, T, Tp, H, d, out_mode, of, oh, ol)
-    if (nblk(32 * AT_QPW * AT_QW) >= n_cu) AT_GO(AT_QW, AT_QPW);
-    else if (nblk(256) >= n_cu) AT_GO(8, 1);
-    else AT_GO(4, 1);
+    const int n1 = (T + 255) / 256, n2 = (T + 511) / 512;
+    const long long bh = (long long)B * H, r1 = (bh * n1 + n_cu - 1) / n_cu, r2 = (bh * n2 + n_cu - 1) / n_cu * 2;
+#define AT_GO(QPW_, NQ_)                                                                                             \
+    hipLaunchKernelGGL(k_attention3<QPW_>, dim3((unsigned)(bh * NQ_)), dim3(512), 0, st, qh, ql, kh, kl, vth, vtl, T, \
+                       Tp, H, d, NQ_, out_mode, of, oh, ol)
+    if (r1 < r2) AT_GO(1, n1);
+    else AT_GO(2, n2);
 #undef AT_GO
 }
