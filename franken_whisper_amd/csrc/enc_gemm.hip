@@ -1,22 +1,16 @@
-// enc_gemm.hip — the encoder's dense contractions on MFMA (gfx950).
+// enc_gemm.hip — the int8 plan's dense contractions on MFMA (gfx950).
 //
-// One tiled GEMM template C[M,N] = A[M,K] x B[N,K]^T serves every encoder
-// linear and the conv stem (as an im2col GEMM).  Operand kinds:
-//   KIND_I8   : i8 x i8 -> i32 (v_mfma_i32_32x32x32_i8).  The int8 plan's
-//               accumulators are exact integers, equal to the reference's
-//               maddubs sum minus 128*colsum (nn.rs:1537-1771) or its i8 dot
-//               (encoder.rs:2524-2606); epilogue ((f32)acc * s_x) * s_w (+ b)
-//               in the reference's association (nn.rs:1660-1700,
-//               encoder.rs:2573-2580).
-//   KIND_F16S : f32 activations carried as an f16 pair (hi, lo = f16(a - hi))
-//               against the f16 weights (exact: the reference dequantizes f16
-//               weights to f32), two v_mfma_f32_32x32x16_f16 per product;
-//               per-product error <= 2^-22 |a| + 2^-25, f32 accumulation.
+// C[M,N] = A[M,K] x B[N,K]^T, i8 x i8 -> i32 (v_mfma_i32_32x32x32_i8).  The
+// accumulators are exact integers, equal to the reference's maddubs sum minus
+// 128*colsum (nn.rs:1537-1771) or its i8 dot (encoder.rs:2524-2606); epilogue
+// ((f32)acc * s_x) * s_w (+ b) in the reference's association
+// (nn.rs:1660-1700, encoder.rs:2573-2580).  (The f16-pair GEMMs are in
+// enc_gemm_f16.hip.)
 //
 // Block = 256 threads as 2x2 waves; block tile BM x BN (128x128 by default;
 // 256x256 and 256x128 for sweeps);
 // each wave owns (BM/2) x (BN/2) as a grid of 32x32 MFMA tiles.  K advances
-// 64 bytes per stage (64 int8 or 32 f16 values); a stage is staged global ->
+// 64 bytes per stage; a stage is staged global ->
 // registers -> LDS (rows padded to 80 bytes: conflict-free 16-byte reads),
 // double buffered with one barrier per stage.  The epilogue is a template
 // parameter so its loops fully unroll and the accumulators stay in registers.
@@ -32,31 +26,9 @@
 #include <cstdlib>
 #include <cstring>
 
-#include "fw_enc.h"
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v4f __attribute__((ext_vector_type(4)));
+#include "enc_gemm.h"
 
 #define GEMM_LDSR 80 // LDS row stride in bytes (64 data + 16 pad)
-
-__device__ __forceinline__ void fw_split2(float v, uint16_t &hi, uint16_t &lo) {
-    asm volatile("" : "+v"(v));
-    _Float16 h = (_Float16)v;
-    float r = v - (float)h;
-    asm volatile("" : "+v"(r));
-    hi = __builtin_bit_cast(uint16_t, h);
-    lo = __builtin_bit_cast(uint16_t, (_Float16)r);
-}
-// The same, or-ing into `of` whether the hi half overflows: |v| >= 65520
-// rounds to an infinite f16 (65504 is the largest finite one), and the pair
-// then carries inf / NaN instead of v.
-__device__ __forceinline__ void fw_split2(float v, uint16_t &hi, uint16_t &lo, uint32_t &of) {
-    of |= fabsf(v) >= 65520.0f ? 1u : 0u;
-    fw_split2(v, hi, lo);
-}
 
 __global__ void __launch_bounds__(256) k_split_f16(const float4 *x, size_t n4, uint2 *hi, uint2 *lo, int *ovf) {
     uint32_t of = 0;
@@ -83,28 +55,14 @@ void fw_launch_split_f16(hipStream_t st, const float *x, size_t n, uint16_t *hi,
 }
 
 // Epilogue for the 4 consecutive rows row0..row0+3 of one column.
-template <int KIND, int EPI>
+template <int EPI>
 __device__ __forceinline__ void gemm_store4(const FwGemm &g, int row0, int col, const float (&a)[4]) {
     if (col >= g.N) return;
-    if constexpr (EPI == FW_EPI_XKV) {
-        const int d = g.ldc, l = col / (2 * d), r = col - l * 2 * d, kv = r >= d ? 1 : 0, c = r - kv * d;
-        const int h = c >> 6, dd = c & 63;
-        const float bias = g.bias ? g.bias[col] : 0.0f;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int row = row0 + e;
-            if (row >= g.M) continue;
-            const int s = row / g.T, t = row - s * g.T;
-            const size_t lh = ((size_t)s * g.L + l) * g.H + h;
-            if (kv == 0) g.o16[0][(lh * g.T + t) * 64 + dd] = fw_f2h(a[e] * g.scale);
-            else g.o16[1][(lh * 64 + dd) * g.T + t] = fw_f2h(a[e] + bias);
-        }
-        return;
-    } else if constexpr (EPI == FW_EPI_QKV) {
+    if constexpr (EPI == FW_EPI_QKV) {
         // head-major split outputs: Q, K as [B, H, T, 64]; V as [B, H, 64, Tp]
         const int d = g.ldc, which = col / d, cc = col - which * d, h = cc >> 6, dd = cc & 63;
         float bias = g.bias ? g.bias[col] : 0.0f;
-        float sw = KIND == FW_KIND_I8 ? g.sw[col] : 1.0f;
+        float sw = g.sw[col];
         float v[4];
         uint16_t hi[4], lo[4];
         uint32_t of = 0;
@@ -112,7 +70,7 @@ __device__ __forceinline__ void gemm_store4(const FwGemm &g, int row0, int col, 
         for (int e = 0; e < 4; e++) {
             int row = row0 + e;
             float x = a[e];
-            if constexpr (KIND == FW_KIND_I8) x = row < g.M ? x * g.sx[row] * sw : 0.0f;
+            x = row < g.M ? x * g.sx[row] * sw : 0.0f;
             if (g.bias) x = x + bias;
             v[e] = x;
             fw_split2(v[e], hi[e], lo[e], of);
@@ -154,36 +112,22 @@ __device__ __forceinline__ void gemm_store4(const FwGemm &g, int row0, int col, 
         return;
     } else {
         float bias = g.bias ? g.bias[col] : 0.0f;
-        float sw = (KIND == FW_KIND_I8 && EPI != FW_EPI_ACC32) ? g.sw[col] : 1.0f;
+        float sw = EPI != FW_EPI_ACC32 ? g.sw[col] : 1.0f;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             int row = row0 + e;
             if (row >= g.M) continue;
             size_t o = (size_t)row * g.ldc + col;
             if constexpr (EPI == FW_EPI_ACC32) {
-                if constexpr (KIND == FW_KIND_I8) ((int *)g.C)[o] = (int)a[e];
-                else g.C[o] = a[e];
+                ((int *)g.C)[o] = (int)a[e];
                 continue;
             } else {
-                float v = a[e];
-                if constexpr (KIND == FW_KIND_I8) v = v * g.sx[row] * sw;
+                float v = a[e] * g.sx[row] * sw;
                 if (g.bias) v = v + bias;
                 if constexpr (EPI == FW_EPI_F32) {
                     g.C[o] = v;
                 } else if constexpr (EPI == FW_EPI_RESID) {
                     g.C[o] = g.C[o] + v;
-                } else if constexpr (EPI == FW_EPI_GELU_F32) {
-                    g.C[o] = fw_gelu(v, g.gelu_tab);
-                } else if constexpr (EPI == FW_EPI_GELU_SPLIT) {
-                    uint16_t hi, lo;
-                    uint32_t of = 0;
-                    fw_split2(fw_gelu(v, g.gelu_tab), hi, lo, of);
-                    if (of && g.ovf) *g.ovf = 1;
-                    g.o16[0][o] = hi;
-                    g.o16[1][o] = lo;
-                } else if constexpr (EPI == FW_EPI_CONV2) {
-                    int t = row % g.T;
-                    g.C[o] = fw_gelu(v, g.gelu_tab) + g.pos[(size_t)t * g.ldc + col];
                 }
             }
         }
@@ -192,23 +136,13 @@ __device__ __forceinline__ void gemm_store4(const FwGemm &g, int row0, int col, 
 
 // Epilogue of a BM x BN block tile: wave (wm, wn) holds TM x TN 32x32
 // accumulator tiles.  `lds` (>= 4 * 32 * 33 floats) is free scratch here.
-// Block id -> tile sequence number.  map 1: the hardware deals blocks
-// round-robin to the 8 XCDs, so block ids are remapped to give each XCD a
-// contiguous run of the tile sequence; map 0: identity.
-__device__ __forceinline__ int gemm_tile_order(int map) {
-    const int nb = gridDim.x, bid = blockIdx.x;
-    if (!map) return bid;
-    const int xcd = bid & 7, loc = bid >> 3, per = nb >> 3, rem = nb & 7;
-    return xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
-}
-
-template <int KIND, int EPI, int BM, int BN, typename accT>
-__device__ __forceinline__ void gemm_epilogue(const FwGemm &g, accT (&acc)[BM / 64][BN / 64], unsigned char *lds,
+template <int EPI, int BM, int BN>
+__device__ __forceinline__ void gemm_epilogue(const FwGemm &g, v16i (&acc)[BM / 64][BN / 64], unsigned char *lds,
                                               int m0, int n0) {
     constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave >> 1, wn = wave & 1;
-    if constexpr (EPI == FW_EPI_QKV || EPI == FW_EPI_CONV2 || EPI == FW_EPI_XKV) {
+    if constexpr (EPI == FW_EPI_QKV) {
         // Heavy epilogues: written once, in a runtime loop over this wave's
         // tiles, reading each tile back from a wave-private LDS slab (a fully
         // unrolled copy of such an epilogue per tile is too large to unroll,
@@ -233,7 +167,7 @@ __device__ __forceinline__ void gemm_epilogue(const FwGemm &g, accT (&acc)[BM / 
                 float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) v[e] = slab[(rl + e) * 33 + (lane & 31)];
-                gemm_store4<KIND, EPI>(g, m0 + wm * WM + i * 32 + rl, col, v);
+                gemm_store4<EPI>(g, m0 + wm * WM + i * 32 + rl, col, v);
             }
             asm volatile("" ::: "memory");
         }
@@ -245,7 +179,7 @@ __device__ __forceinline__ void gemm_epilogue(const FwGemm &g, accT (&acc)[BM / 
         for (int j = 0; j < TN; j++) {
             const int col = n0 + wn * WN + j * 32 + (lane & 31);
             const int rb = m0 + wm * WM + i * 32 + (lane >> 5) * 4; // + q*8 + e
-            if constexpr (KIND == FW_KIND_I8 && EPI == FW_EPI_ACC32) {
+            if constexpr (EPI == FW_EPI_ACC32) {
                 // exact i32 accumulators: store the integers themselves
                 if (col < g.N)
 #pragma unroll
@@ -259,21 +193,20 @@ __device__ __forceinline__ void gemm_epilogue(const FwGemm &g, accT (&acc)[BM / 
                 // first store, so the tile waits on memory once, not per element.
                 const int colc = col < g.N ? col : g.N - 1;
                 const float bias = g.bias ? g.bias[colc] : 0.0f;
-                const float sw = KIND == FW_KIND_I8 ? g.sw[colc] : 1.0f;
+                const float sw = g.sw[colc];
                 float sx[16], cv[16];
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
                     int row = rb + (r >> 2) * 8 + (r & 3);
                     row = row < g.M ? row : g.M - 1;
-                    if constexpr (KIND == FW_KIND_I8) sx[r] = g.sx[row];
+                    sx[r] = g.sx[row];
                     if constexpr (EPI == FW_EPI_RESID) cv[r] = g.C[(size_t)row * g.ldc + colc];
                 }
                 if (col < g.N) {
 #pragma unroll
                     for (int r = 0; r < 16; r++) {
                         const int row = rb + (r >> 2) * 8 + (r & 3);
-                        float v = (float)acc[i][j][r];
-                        if constexpr (KIND == FW_KIND_I8) v = v * sx[r] * sw;
+                        float v = (float)acc[i][j][r] * sx[r] * sw;
                         if (g.bias) v = v + bias;
                         if (row < g.M) {
                             const size_t o = (size_t)row * g.ldc + col;
@@ -281,15 +214,6 @@ __device__ __forceinline__ void gemm_epilogue(const FwGemm &g, accT (&acc)[BM / 
                                 g.C[o] = v;
                             } else if constexpr (EPI == FW_EPI_RESID) {
                                 g.C[o] = cv[r] + v;
-                            } else if constexpr (EPI == FW_EPI_GELU_F32) {
-                                g.C[o] = fw_gelu(v, g.gelu_tab);
-                            } else if constexpr (EPI == FW_EPI_GELU_SPLIT) {
-                                uint16_t hi, lo;
-                                uint32_t of = 0;
-                                fw_split2(fw_gelu(v, g.gelu_tab), hi, lo, of);
-                                if (of && g.ovf) *g.ovf = 1;
-                                g.o16[0][o] = hi;
-                                g.o16[1][o] = lo;
                             }
                         }
                     }
@@ -298,15 +222,13 @@ __device__ __forceinline__ void gemm_epilogue(const FwGemm &g, accT (&acc)[BM / 
         }
 }
 
-template <int KIND, int EPI, int BM, int BN>
+template <int EPI, int BM, int BN>
 __global__ void __launch_bounds__(256) k_gemm(FwGemm g, int ntm, int ntn) {
-    constexpr int NA = KIND == FW_KIND_F16S ? 2 : 1;
-    constexpr int ES = KIND == FW_KIND_I8 ? 1 : 2;
     constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-    constexpr int ROWS = NA * BM + BN; // LDS rows per stage
+    constexpr int ROWS = BM + BN; // LDS rows per stage
     constexpr int STAGE = ROWS * GEMM_LDSR;
     constexpr int CH = ROWS * 4 / 256; // 16-byte chunks per thread per stage
-    constexpr int CHA = NA * BM / 64;  // chunks (per thread) that belong to A
+    constexpr int CHA = BM / 64;  // chunks (per thread) that belong to A
     __shared__ __align__(16) unsigned char lds[2 * STAGE];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
@@ -317,7 +239,7 @@ __global__ void __launch_bounds__(256) k_gemm(FwGemm g, int ntm, int ntn) {
     const int gsize = GM * ntn, grp = t / gsize, first_m = grp * GM;
     const int gm = min(ntm - first_m, GM), rr = t - grp * gsize;
     const int m0 = (first_m + rr % gm) * BM, n0 = (rr / gm) * BN;
-    const int nsteps = g.K * ES / 64;
+    const int nsteps = g.K / 64;
 
     int4 stg[CH];
     auto gload = [&](int s) {
@@ -326,12 +248,12 @@ __global__ void __launch_bounds__(256) k_gemm(FwGemm g, int ntm, int ntn) {
             const int row = (tid >> 2) + q * 64, cc = tid & 3;
             const size_t koff = (size_t)s * 64 + cc * 16;
             if (q < CHA) {
-                const int a = (q * 64) / BM, r = row - a * BM, gr = m0 + r;
-                const unsigned char *base = (const unsigned char *)(a == 0 ? g.A : g.A2);
-                stg[q] = gr < g.M ? *(const int4 *)(base + (size_t)gr * g.lda * ES + koff) : make_int4(0, 0, 0, 0);
+                const int gr = m0 + row;
+                const unsigned char *base = (const unsigned char *)g.A;
+                stg[q] = gr < g.M ? *(const int4 *)(base + (size_t)gr * g.lda + koff) : make_int4(0, 0, 0, 0);
             } else {
-                const int gn = n0 + row - NA * BM;
-                stg[q] = gn < g.N ? *(const int4 *)((const unsigned char *)g.B + (size_t)gn * g.ldb * ES + koff)
+                const int gn = n0 + row - BM;
+                stg[q] = gn < g.N ? *(const int4 *)((const unsigned char *)g.B + (size_t)gn * g.ldb + koff)
                                   : make_int4(0, 0, 0, 0);
             }
         }
@@ -345,8 +267,7 @@ __global__ void __launch_bounds__(256) k_gemm(FwGemm g, int ntm, int ntn) {
         }
     };
 
-    typedef typename std::conditional<KIND == FW_KIND_I8, v16i, v16f>::type accT;
-    accT acc[TM][TN];
+    v16i acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -364,39 +285,29 @@ __global__ void __launch_bounds__(256) k_gemm(FwGemm g, int ntm, int ntn) {
 #pragma unroll
         for (int ks = 0; ks < 2; ks++) {
             const int koff = ks * 32 + (lane >> 5) * 16;
-            v4i af[NA][TM], bf[TN];
+            v4i af[TM], bf[TN];
 #pragma unroll
             for (int i = 0; i < TM; i++) {
                 const int row = wm * WM + i * 32 + (lane & 31);
-#pragma unroll
-                for (int a = 0; a < NA; a++) af[a][i] = *(const v4i *)(tb + (a * BM + row) * GEMM_LDSR + koff);
+                af[i] = *(const v4i *)(tb + row * GEMM_LDSR + koff);
             }
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 const int row = wn * WN + j * 32 + (lane & 31);
-                bf[j] = *(const v4i *)(tb + (NA * BM + row) * GEMM_LDSR + koff);
+                bf[j] = *(const v4i *)(tb + (BM + row) * GEMM_LDSR + koff);
             }
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < TN; j++) {
-                    if constexpr (KIND == FW_KIND_I8) {
-                        acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[0][i], bf[j], acc[i][j], 0, 0, 0);
-                    } else {
-                        const v8h bh = __builtin_bit_cast(v8h, bf[j]);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, af[0][i]), bh,
-                                                                           acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, af[1][i]), bh,
-                                                                           acc[i][j], 0, 0, 0);
-                    }
-                }
+                for (int j = 0; j < TN; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], acc[i][j], 0, 0, 0);
         }
         if (s + 1 < nsteps) lstore(buf ^ 1);
         __syncthreads();
         buf ^= 1;
     }
 
-    gemm_epilogue<KIND, EPI, BM, BN>(g, acc, lds, m0, n0);
+    gemm_epilogue<EPI, BM, BN>(g, acc, lds, m0, n0);
 }
 
 // ---------------------------------------------------------------------------
@@ -406,15 +317,12 @@ __global__ void __launch_bounds__(256) k_gemm(FwGemm g, int ntm, int ntn) {
 // XOR-swizzled by (r ^ r>>2) & 3, so the MFMA fragment reads are free of bank
 // conflicts.  Each wave loads ROWS/64 row groups of 16 rows per stage (one
 // instruction writes 16 rows x 64 bytes = 1 KB contiguous in LDS).
-__device__ __forceinline__ int gsw(int r) { return (r ^ (r >> 2)) & 3; }
 
 
-template <int KIND, int EPI, int BM, int BN, int NS>
+template <int EPI, int BM, int BN, int NS>
 __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
-    constexpr int NA = KIND == FW_KIND_F16S ? 2 : 1;
-    constexpr int ES = KIND == FW_KIND_I8 ? 1 : 2;
     constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-    constexpr int ROWS = NA * BM + BN;
+    constexpr int ROWS = BM + BN;
     constexpr int STAGE = ROWS * 64;
     constexpr int LPW = ROWS / 64; // load instructions per wave per stage
     __shared__ __align__(1024) unsigned char lds[NS * STAGE];
@@ -426,7 +334,7 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
     const int gsize = GM * ntn, grp = t / gsize, first_m = grp * GM;
     const int gm = min(ntm - first_m, GM), rr = t - grp * gsize;
     const int m0 = (first_m + rr % gm) * BM, n0 = (rr / gm) * BN;
-    const int nsteps = g.K * ES / 64;
+    const int nsteps = g.K / 64;
 
     // per-lane source rows of this wave's row groups (fixed over k)
     const unsigned char *src[LPW];
@@ -434,15 +342,14 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
     for (int q = 0; q < LPW; q++) {
         const int lr = (wave * LPW + q) * 16 + (lane >> 2); // LDS row
         const int c = (lane & 3) ^ gsw(lr);                  // global chunk for this LDS slot
-        if (lr < NA * BM) {
-            const int a = lr / BM, r = lr - a * BM;
-            int gr = m0 + r;
+        if (lr < BM) {
+            int gr = m0 + lr;
             gr = gr < g.M ? gr : g.M - 1; // rows past M: in-bounds reload, never stored
-            src[q] = (const unsigned char *)(a == 0 ? g.A : g.A2) + (size_t)gr * g.lda * ES + c * 16;
+            src[q] = (const unsigned char *)g.A + (size_t)gr * g.lda + c * 16;
         } else {
-            int gn = n0 + lr - NA * BM;
+            int gn = n0 + lr - BM;
             gn = gn < g.N ? gn : g.N - 1;
-            src[q] = (const unsigned char *)g.B + (size_t)gn * g.ldb * ES + c * 16;
+            src[q] = (const unsigned char *)g.B + (size_t)gn * g.ldb + c * 16;
         }
     }
     auto issue = [&](int s) {
@@ -454,8 +361,7 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
                                              (void __attribute__((address_space(3))) *)(dst + q * 1024), 16, 0, 0);
     };
 
-    typedef typename std::conditional<KIND == FW_KIND_I8, v16i, v16f>::type accT;
-    accT acc[TM][TN];
+    v16i acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -467,20 +373,18 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
     // sets 0 and 1; the next substep's LDS reads are issued before the current
     // substep's MFMAs, so fragment latency hides behind MFMA issue.  The stage
     // barrier sits between the substeps of a stage.
-    v4i fa[2][NA][TM], fb[2][TN];
+    v4i fa[2][TM], fb[2][TN];
     auto ldfrag = [&](int set, int stage, int ks) {
         const unsigned char *tb = lds + (stage % NS) * STAGE;
         const int c = ks * 2 + (lane >> 5);
 #pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int a = 0; a < NA; a++) {
-                const int lr = a * BM + wm * WM + i * 32 + (lane & 31);
-                fa[set][a][i] = *(const v4i *)(tb + lr * 64 + ((c ^ gsw(lr)) << 4));
-            }
+        for (int i = 0; i < TM; i++) {
+            const int lr = wm * WM + i * 32 + (lane & 31);
+            fa[set][i] = *(const v4i *)(tb + lr * 64 + ((c ^ gsw(lr)) << 4));
+        }
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-            const int lr = NA * BM + wn * WN + j * 32 + (lane & 31);
+            const int lr = BM + wn * WN + j * 32 + (lane & 31);
             fb[set][j] = *(const v4i *)(tb + lr * 64 + ((c ^ gsw(lr)) << 4));
         }
     };
@@ -488,17 +392,8 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) {
-                if constexpr (KIND == FW_KIND_I8) {
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[set][0][i], fb[set][j], acc[i][j], 0, 0, 0);
-                } else {
-                    const v8h bh = __builtin_bit_cast(v8h, fb[set][j]);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, fa[set][0][i]), bh,
-                                                                       acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, fa[set][1][i]), bh,
-                                                                       acc[i][j], 0, 0, 0);
-                }
-            }
+            for (int j = 0; j < TN; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[set][i], fb[set][j], acc[i][j], 0, 0, 0);
     };
 
 #pragma unroll
@@ -529,7 +424,7 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
     }
     FW_WAIT_VM(0);
     __syncthreads(); // LDS is reused by the heavy epilogues
-    gemm_epilogue<KIND, EPI, BM, BN>(g, acc, lds, m0, n0);
+    gemm_epilogue<EPI, BM, BN>(g, acc, lds, m0, n0);
 }
 
 // ---------------------------------------------------------------------------
@@ -861,13 +756,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_pi8(FwGemm g, int ntm, 
                     }
                 }
         } else if constexpr (QKV) {
-            // Q, K: [B, H, T, 64] f16 hi/lo rows, written through a wave-private
-            // LDS slab so each lane stores 16 consecutive dims (32-byte runs).
-            // V^T: [B, H, 64, Tp] at key positions fw_vt_pos(t); a lane's 8
-            // values r = 8c .. 8c+7 sit at 8 consecutive positions (window
-            // tiles start at multiples of 32), so they go out as 16-byte runs.
             float *slab = (float *)(lds + NS * STAGE + 2 * SCLN * 4 + wave * SLABB);
-            const int d = g.ldc, wnd = m0 / g.T, tb0 = m0 - wnd * g.T;
+            const int wnd = m0 / g.T, tb0 = m0 - wnd * g.T;
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -886,76 +776,12 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_pi8(FwGemm g, int ntm, 
                         if (has_bias) v[r] = v[r] + bb;
                     }
                     if (c0 >= g.N) continue;
-                    const int which = c0 / d, cc = c0 - which * d, h = cc >> 6, dd0 = cc & 63;
                     const int t0 = tb0 + wm * WM + i * 32; // window position of the tile's first row
                     const int vrows = mrows - (wm * WM + i * 32);
                     if (vrows <= 0) continue;
-                    if (which == 2) {
-                        const int dd = dd0 + (ln & 31);
-                        uint16_t *vh = g.o16[4] + (((size_t)wnd * g.H + h) * 64 + dd) * g.Tp;
-                        uint16_t *vl = g.o16[5] + (((size_t)wnd * g.H + h) * 64 + dd) * g.Tp;
-#pragma unroll
-                        for (int c = 0; c < 2; c++) {
-                            const int pb = t0 + 16 * c + 8 * (ln >> 5); // first of 8 positions
-                            uint16_t hi[8], lo[8];
-#pragma unroll
-                            for (int e = 0; e < 8; e++) fw_split2(v[8 * c + e], hi[e], lo[e], ovf_any);
-                            if (16 * c + 16 <= vrows) {
-                                uint4 ph, pl;
-                                ph.x = hi[0] | ((uint32_t)hi[1] << 16);
-                                ph.y = hi[2] | ((uint32_t)hi[3] << 16);
-                                ph.z = hi[4] | ((uint32_t)hi[5] << 16);
-                                ph.w = hi[6] | ((uint32_t)hi[7] << 16);
-                                pl.x = lo[0] | ((uint32_t)lo[1] << 16);
-                                pl.y = lo[2] | ((uint32_t)lo[3] << 16);
-                                pl.z = lo[4] | ((uint32_t)lo[5] << 16);
-                                pl.w = lo[6] | ((uint32_t)lo[7] << 16);
-                                *(uint4 *)(vh + pb) = ph;
-                                *(uint4 *)(vl + pb) = pl;
-                            } else {
-#pragma unroll
-                                for (int e = 0; e < 8; e++) {
-                                    // value e is key t0 + 16c + 8*(e/4) + 4*(lane/32) + e%4
-                                    const int rr = 16 * c + 8 * (e >> 2) + 4 * (ln >> 5) + (e & 3);
-                                    if (rr < vrows) {
-                                        const int p = fw_vt_pos(t0 + rr);
-                                        vh[p] = hi[e];
-                                        vl[p] = lo[e];
-                                    }
-                                }
-                            }
-                        }
-                    } else {
-                        // the slab is private to this wave and a wave's LDS accesses
-                        // run in order: only the compiler must not reorder them
-                        asm volatile("" ::: "memory");
-#pragma unroll
-                        for (int r = 0; r < 16; r++)
-                            slab[((r >> 2) * 8 + (ln >> 5) * 4 + (r & 3)) * 40 + (ln & 31)] = v[r];
-                        asm volatile("" ::: "memory");
-                        const int row = ln >> 1, half = ln & 1;
-                        v4f w4[4];
-#pragma unroll
-                        for (int q = 0; q < 4; q++) w4[q] = *(const v4f *)(slab + row * 40 + half * 16 + q * 4);
-                        asm volatile("" ::: "memory");
-                        if (row < vrows) {
-                            uint32_t ph[8], pl[8];
-#pragma unroll
-                            for (int q = 0; q < 8; q++) {
-                                uint16_t h0, l0, h1, l1;
-                                fw_split2(w4[q >> 1][(q & 1) * 2], h0, l0, ovf_any);
-                                fw_split2(w4[q >> 1][(q & 1) * 2 + 1], h1, l1, ovf_any);
-                                ph[q] = h0 | ((uint32_t)h1 << 16);
-                                pl[q] = l0 | ((uint32_t)l1 << 16);
-                            }
-                            const size_t o = (((size_t)wnd * g.H + h) * g.T + t0 + row) * 64 + dd0 + half * 16;
-                            uint4 *qh = (uint4 *)(g.o16[2 * which] + o), *ql = (uint4 *)(g.o16[2 * which + 1] + o);
-                            qh[0] = make_uint4(ph[0], ph[1], ph[2], ph[3]);
-                            qh[1] = make_uint4(ph[4], ph[5], ph[6], ph[7]);
-                            ql[0] = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-                            ql[1] = make_uint4(pl[4], pl[5], pl[6], pl[7]);
-                        }
-                    }
+                    int lt = ln; // opaque per tile: addresses are not hoisted over the tiles
+                    asm volatile("" : "+v"(lt));
+                    qkv_store32(g, slab, v, lt, c0, wnd, t0, vrows, ovf_any);
                 }
         }
 #pragma unroll
@@ -1005,31 +831,30 @@ static int pick_tile(int M, int N, int ncu) {
     return 7;
 }
 
-template <int KIND, int EPI, int BM, int BN>
+template <int EPI, int BM, int BN>
 static void launch_one(hipStream_t st, const FwGemm &g) {
     int ntm = (g.M + BM - 1) / BM, ntn = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL((k_gemm<KIND, EPI, BM, BN>), dim3(ntm * ntn), dim3(256), 0, st, g, ntm, ntn);
+    hipLaunchKernelGGL((k_gemm<EPI, BM, BN>), dim3(ntm * ntn), dim3(256), 0, st, g, ntm, ntn);
 }
 
-template <int KIND, int EPI, int BM, int BN, int NS>
+template <int EPI, int BM, int BN, int NS>
 static void launch_pipe(hipStream_t st, const FwGemm &g) {
     int ntm = (g.M + BM - 1) / BM, ntn = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL((k_gemm2<KIND, EPI, BM, BN, NS>), dim3(ntm * ntn), dim3(256), 0, st, g, ntm, ntn);
+    hipLaunchKernelGGL((k_gemm2<EPI, BM, BN, NS>), dim3(ntm * ntn), dim3(256), 0, st, g, ntm, ntn);
 }
 
-template <int KIND, int EPI>
+template <int EPI>
 static void launch_tiles(hipStream_t st, const FwGemm &g, int tile) {
-    constexpr int NSB = KIND == FW_KIND_I8 ? 4 : 3; // stages of the 256-row pipelined tiles (LDS <= 160 KB)
     switch (tile) {
-    case 0: launch_one<KIND, EPI, 256, 256>(st, g); break;
-    case 1: launch_one<KIND, EPI, 256, 128>(st, g); break;
-    case 2: launch_one<KIND, EPI, 128, 128>(st, g); break;
-    case 3: launch_pipe<KIND, EPI, 256, 256, NSB>(st, g); break;
-    case 4: launch_pipe<KIND, EPI, 256, 128, NSB>(st, g); break;
-    case 5: launch_pipe<KIND, EPI, 128, 128, 4>(st, g); break;
-    case 6: launch_pipe<KIND, EPI, 256, 128, 2>(st, g); break;
-    case 7: launch_pipe<KIND, EPI, 128, 128, 3>(st, g); break;
-    default: launch_pipe<KIND, EPI, 128, 128, 2>(st, g); break;
+    case 0: launch_one<EPI, 256, 256>(st, g); break;
+    case 1: launch_one<EPI, 256, 128>(st, g); break;
+    case 2: launch_one<EPI, 128, 128>(st, g); break;
+    case 3: launch_pipe<EPI, 256, 256, 4>(st, g); break;
+    case 4: launch_pipe<EPI, 256, 128, 4>(st, g); break;
+    case 5: launch_pipe<EPI, 128, 128, 4>(st, g); break;
+    case 6: launch_pipe<EPI, 256, 128, 2>(st, g); break;
+    case 7: launch_pipe<EPI, 128, 128, 3>(st, g); break;
+    default: launch_pipe<EPI, 128, 128, 2>(st, g); break;
     }
 }
 
@@ -1083,12 +908,13 @@ bool fw_launch_gemm(hipStream_t st, int kind, const FwGemm &g0) {
         const char *e = getenv("FWHIP_GEMM_I8P");
         pi8 = e ? atoi(e) : 1;
     }
+    if (kind == FW_KIND_F16S) return fw_launch_gemm_f16(st, g0, ncu);
     // One window (M <= 1536 rows) fills the CUs better with the one-tile-per-
     // block kernels' tiles: the persistent kernel's 256 x 256 tiles give the
     // q/k/v GEMM 90 tiles for 256 CUs (one-window encoder pass 8.35 -> 7.78
     // ms; from two windows on the persistent kernel is faster: 9.81 against
     // 10.15 ms, ten 36.1 against 40.3).  Both routes give the same bits.
-    if (kind == FW_KIND_I8 && pi8 && g.M > 1536 && g.K % 64 == 0 &&
+    if (pi8 && g.M > 1536 && g.K % 64 == 0 &&
         (g.epi != FW_EPI_QKV || (g.T > 0 && g.M % g.T == 0))) {
         switch (g.epi) {
         case FW_EPI_F32: launch_pi8_tiles<FW_EPI_F32>(st, g, ncu); return true;
@@ -1100,24 +926,11 @@ bool fw_launch_gemm(hipStream_t st, int kind, const FwGemm &g0) {
         }
     }
     int tile = pick_tile(g.M, g.N, ncu);
-    if (kind == FW_KIND_I8) {
-        switch (g.epi) {
-        case FW_EPI_F32: launch_tiles<FW_KIND_I8, FW_EPI_F32>(st, g, tile); return true;
-        case FW_EPI_RESID: launch_tiles<FW_KIND_I8, FW_EPI_RESID>(st, g, tile); return true;
-        case FW_EPI_QKV: launch_tiles<FW_KIND_I8, FW_EPI_QKV>(st, g, tile); return true;
-        case FW_EPI_ACC32: launch_tiles<FW_KIND_I8, FW_EPI_ACC32>(st, g, tile); return true;
-        default: return false;
-        }
-    } else {
-        switch (g.epi) {
-        case FW_EPI_F32: launch_tiles<FW_KIND_F16S, FW_EPI_F32>(st, g, tile); return true;
-        case FW_EPI_RESID: launch_tiles<FW_KIND_F16S, FW_EPI_RESID>(st, g, tile); return true;
-        case FW_EPI_GELU_F32: launch_tiles<FW_KIND_F16S, FW_EPI_GELU_F32>(st, g, tile); return true;
-        case FW_EPI_GELU_SPLIT: launch_tiles<FW_KIND_F16S, FW_EPI_GELU_SPLIT>(st, g, tile); return true;
-        case FW_EPI_CONV2: launch_tiles<FW_KIND_F16S, FW_EPI_CONV2>(st, g, tile); return true;
-        case FW_EPI_QKV: launch_tiles<FW_KIND_F16S, FW_EPI_QKV>(st, g, tile); return true;
-        case FW_EPI_XKV: launch_tiles<FW_KIND_F16S, FW_EPI_XKV>(st, g, tile); return true;
-        default: return false;
-        }
+    switch (g.epi) {
+    case FW_EPI_F32: launch_tiles<FW_EPI_F32>(st, g, tile); return true;
+    case FW_EPI_RESID: launch_tiles<FW_EPI_RESID>(st, g, tile); return true;
+    case FW_EPI_QKV: launch_tiles<FW_EPI_QKV>(st, g, tile); return true;
+    case FW_EPI_ACC32: launch_tiles<FW_EPI_ACC32>(st, g, tile); return true;
+    default: return false;
     }
 }

@@ -484,25 +484,46 @@ __global__ void __launch_bounds__(1024) k_gelu_quant_h16(const uint16_t *hx, con
     }
 }
 
-// im2col for conv1d (kernel 3, pad 1; conv1d_wt nn.rs:5006-5103) into the f16
-// pair the GEMM consumes.  Column order kk*Cin + ci (weights are reordered to
-// match at load); columns >= 3*Cin are zero padding up to Kp.
-__global__ void k_im2col(const float *x, int B, int Tin, int Cin, int stride, int Tout, int Kp, uint16_t *hi,
-                         uint16_t *lo, int *ovf) {
-    size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t total = (size_t)B * Tout * Kp;
-    if (idx >= total) return;
-    int col = (int)(idx % Kp);
-    size_t row = idx / Kp;
-    int b = (int)(row / Tout), t = (int)(row % Tout);
-    float v = 0.0f;
-    if (col < 3 * Cin) {
-        int kk = col / Cin, ci = col % Cin;
-        int ti = t * stride + kk - 1;
-        if (ti >= 0 && ti < Tin) v = x[((size_t)b * Tin + ti) * Cin + ci];
+// im2col for conv1 (kernel 3, pad 1, stride 1; conv1d_wt nn.rs:5006-5103) into the
+// f16 pair the GEMM consumes.  Column order kk*Cin + ci (weights are reordered
+// to match at load), so row t is the 3 Cin values from x[t - 1] on; columns >=
+// 3*Cin are zero padding up to Kp (a multiple of 8).  A thread makes 8 columns
+// (16-byte stores).  The blocks past them zero the padding rows of conv1's
+// output (conv2 reads that output in place: its rows 2t-1 .. 2t+1 are one run
+// of 3 d values, so its im2col is the output itself at a row stride of 2 d).
+__global__ void __launch_bounds__(256) k_im2col(const float *x, int B, int T, int Cin, int Kp, uint4 *hi, uint4 *lo,
+                                                int *ovf, uint4 *oh, uint4 *ol, int d, int *lo_any, int nblk) {
+    if ((int)blockIdx.x >= nblk) {
+        const int n8 = d >> 3, total = B * 2 * n8;
+        if ((int)blockIdx.x == nblk && threadIdx.x == 0) *lo_any = 0;
+        for (int i = (blockIdx.x - nblk) * 256 + threadIdx.x; i < total; i += (gridDim.x - nblk) * 256) {
+            const int r = i / n8, c = i - r * n8;
+            const size_t o = ((size_t)(r >> 1) * (T + 2) + (r & 1) * (T + 1)) * n8 + c;
+            oh[o] = make_uint4(0, 0, 0, 0);
+            ol[o] = make_uint4(0, 0, 0, 0);
+        }
+        return;
     }
+    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const int k8 = Kp >> 3;
+    const size_t row = idx / k8;
+    if (row >= (size_t)B * T) return;
+    const int col = (int)(idx - row * k8) * 8, b = (int)(row / T), t = (int)(row - (size_t)b * T);
+    const float *w = x + (size_t)b * T * Cin; // the window; element f0 + e is column col + e of row t
+    const int f0 = (t - 1) * Cin + col, n = T * Cin;
+    uint16_t h[8], l[8];
     uint32_t of = 0;
-    fw_split(v, hi[idx], lo[idx], of);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const int f = f0 + e;
+        const bool in = col + e < 3 * Cin && f >= 0 && f < n;
+        const float v = w[in ? f : 0];
+        fw_split(in ? v : 0.0f, h[e], l[e], of);
+    }
+    hi[idx] = make_uint4(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16), h[4] | ((uint32_t)h[5] << 16),
+                         h[6] | ((uint32_t)h[7] << 16));
+    lo[idx] = make_uint4(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16), l[4] | ((uint32_t)l[5] << 16),
+                         l[6] | ((uint32_t)l[7] << 16));
     if (of && ovf) *ovf = 1;
 }
 
@@ -1175,11 +1196,12 @@ bool fw_launch_gelu_quant_h16(hipStream_t st, const uint16_t *hx, const float *s
     }
 #undef GQH
 }
-void fw_launch_im2col(hipStream_t st, const float *x, int B, int Tin, int Cin, int stride, int Tout, int Kp,
-                      uint16_t *hi, uint16_t *lo, int *ovf) {
-    size_t total = (size_t)B * Tout * Kp;
-    hipLaunchKernelGGL(k_im2col, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, x, B, Tin, Cin, stride,
-                       Tout, Kp, hi, lo, ovf);
+void fw_launch_im2col(hipStream_t st, const float *x, int B, int T, int Cin, int Kp, uint16_t *hi, uint16_t *lo,
+                      int *ovf, uint16_t *oh, uint16_t *ol, int d, int *lo_any) {
+    const size_t total = (size_t)B * T * (Kp / 8);
+    const int nblk = (int)((total + 255) / 256), npad = (B * 2 * (d / 8) + 255) / 256;
+    hipLaunchKernelGGL(k_im2col, dim3((unsigned)(nblk + npad)), dim3(256), 0, st, x, B, T, Cin, Kp, (uint4 *)hi,
+                       (uint4 *)lo, ovf, (uint4 *)oh, (uint4 *)ol, d, lo_any, nblk);
 }
 void fw_launch_mel_window(hipStream_t st, const float *mel, int n_mel, long long mel_frames, const long long *offs,
                           int n_frames, float *out, int B) {

@@ -27,11 +27,15 @@ struct EncLayerDev {
 
 struct EncBufs {
     int B = 0, nf = 0;
-    float *mel_tm, *a1, *x, *att, *ff;
-    uint16_t *a1h, *a1l, *a2h, *a2l, *hh, *hl, *qh, *ql, *kh, *kl, *vth, *vtl, *ath, *atl, *gh, *gl;
+    float *mel_tm, *x, *att, *ff;
+    uint16_t *a1h, *a1l, *c1h, *c1l, *hh, *hl, *qh, *ql, *kh, *kl, *vth, *vtl, *ath, *atl, *gh, *gl;
     int8_t *hq, *aq, *gq;
     float *hs, *as, *gs;
     long long *offs;
+    // f16-pair GELU outputs: which lo halves are nonzero (FwGemm::lo_in / lo_any), 16 zero bytes
+    uint8_t *lo;
+    int *lo_any;
+    void *zero;
     // ToMe: merged rows, unmerge map, merge workspace
     float *xm;
     int32_t *umap, *umap2; // original row -> current row; the latest merge's map
@@ -233,9 +237,11 @@ static bool ensure_bufs(fwhip_encoder *e, int B, int nf) {
     b.mel_tm = (float *)A(sizeof(float) * M1 * e->nmel);
     b.a1h = (uint16_t *)A(2 * M1 * e->Kp1);
     b.a1l = (uint16_t *)A(2 * M1 * e->Kp1);
-    b.a1 = (float *)A(4 * M1 * d);
-    b.a2h = (uint16_t *)A(2 * M * 3 * d);
-    b.a2l = (uint16_t *)A(2 * M * 3 * d);
+    b.c1h = (uint16_t *)A(2 * (M1 + 2 * (size_t)B) * d); // conv1's output, a zero row before and after each window
+    b.c1l = (uint16_t *)A(2 * (M1 + 2 * (size_t)B) * d);
+    b.lo = (uint8_t *)A((M + 63) / 64 * 128 + 64);
+    b.lo_any = (int *)(b.lo ? b.lo + (M + 63) / 64 * 128 : nullptr);
+    b.zero = b.lo ? b.lo + (M + 63) / 64 * 128 + 16 : nullptr;
     b.x = (float *)A(4 * M * d);
     b.hh = (uint16_t *)A(2 * M * d);
     b.hl = (uint16_t *)A(2 * M * d);
@@ -268,6 +274,7 @@ static bool ensure_bufs(fwhip_encoder *e, int B, int nf) {
     // V^T padding columns (keys >= T) must be finite zeros
     fw_launch_fill_u16(e->ctx->stream, b.vth, vt, 0);
     fw_launch_fill_u16(e->ctx->stream, b.vtl, vt, 0);
+    fw_launch_fill_u16(e->ctx->stream, (uint16_t *)b.lo, ((M + 63) / 64 * 128 + 64) / 2, 0);
     return hipStreamSynchronize(e->ctx->stream) == hipSuccess;
 }
 
@@ -371,18 +378,28 @@ static fwhip_status enc_run(fwhip_encoder *e, int B, int nf, float *out_dev, fwh
     int *ovf = c->ovf_dev;
     fw_ovf_clear(c);
     // conv stem (encoder.rs:1550-1572): conv1 + GELU, conv2 (stride 2) + GELU, + pos_emb
-    fw_launch_im2col(st, b.mel_tm, B, T1, e->nmel, 1, T1, e->Kp1, b.a1h, b.a1l, ovf);
+    fw_launch_im2col(st, b.mel_tm, B, T1, e->nmel, e->Kp1, b.a1h, b.a1l, ovf, b.c1h, b.c1l, d, b.lo_any);
     {
-        FwGemm g = gemm_args(b.a1h, b.a1l, e->conv1w, M1, d, e->Kp1, nullptr, nullptr, e->conv1b, FW_EPI_GELU_F32,
-                             b.a1, d);
+        FwGemm g = gemm_args(b.a1h, b.a1l, e->conv1w, M1, d, e->Kp1, nullptr, nullptr, e->conv1b, FW_EPI_GELU_SPLIT,
+                             nullptr, d);
         g.gelu_tab = gt;
+        g.o16[0] = b.c1h;
+        g.o16[1] = b.c1l;
+        g.T = T1;
+        g.opad = 2;
+        g.lo_any_out = b.lo_any;
+        g.ovf = ovf;
         fw_timed_begin(c, FWHIP_K_ENC_GEMM_F32, 2.0 * M1 * d * 3.0 * e->nmel, &ev);
         fw_launch_gemm(st, FW_KIND_F16S, g);
         fw_timed_end(c, &ev);
     }
-    fw_launch_im2col(st, b.a1, B, T1, d, 2, T2, 3 * d, b.a2h, b.a2l, ovf);
     {
-        FwGemm g = gemm_args(b.a2h, b.a2l, e->conv2w, M, d, 3 * d, nullptr, nullptr, e->conv2b, FW_EPI_CONV2, b.x, d);
+        // row t of a window: conv1's rows 2t-1 .. 2t+1, one run of 3d values
+        FwGemm g = gemm_args(b.c1h, b.c1l, e->conv2w, M, d, 3 * d, nullptr, nullptr, e->conv2b, FW_EPI_CONV2, b.x, d);
+        g.lda = 2 * d;
+        g.apad = 1;
+        g.lo_any = b.lo_any;
+        g.zero = b.zero;
         g.gelu_tab = gt;
         g.pos = e->pos;
         g.T = T2;
@@ -454,11 +471,14 @@ static fwhip_status enc_run(fwhip_encoder *e, int B, int nf, float *out_dev, fwh
             g.gelu_tab = gt;
             g.o16[0] = b.gh;
             g.o16[1] = b.gl;
+            g.lo_out = b.lo;
             g.ovf = ovf;
             fw_timed_begin(c, gcls, 2.0 * Mc * (double)dff * d, &ev);
             fw_launch_gemm(st, kind, g);
             fw_timed_end(c, &ev);
             g = gemm_args(b.gh, b.gl, l.fc2_16, Mc, d, dff, nullptr, nullptr, l.fc2_b, FW_EPI_RESID, X, d);
+            g.lo_in = b.lo;
+            g.zero = b.zero;
         }
         fw_timed_begin(c, gcls, 2.0 * Mc * (double)d * dff, &ev);
         fw_launch_gemm(st, kind, g);

@@ -9,8 +9,7 @@
 
 #define FW_EPI_F32 0
 #define FW_EPI_RESID 1
-#define FW_EPI_GELU_F32 2
-#define FW_EPI_GELU_SPLIT 3
+#define FW_EPI_GELU_SPLIT 3 // f16-pair only, as CONV2
 #define FW_EPI_CONV2 4
 #define FW_EPI_QKV 5
 #define FW_EPI_ACC32 6
@@ -55,6 +54,23 @@ struct FwGemm {
     int L;       // FW_EPI_XKV: decoder layers
     float scale; // FW_EPI_XKV: the key scale
     int map;     // tile order (set by fw_launch_gemm)
+    // f16-pair A operand with extra rows: GEMM row r reads A row r + (r / T) * apad
+    // (windows of T rows, apad rows after each; lda may overlap rows)
+    int apad;
+    // GELU split output row of GEMM row r: r, or with opad r + (r / T) * opad + 1
+    int opad;
+    // Which lo halves of A can be nonzero.  lo_in (nullable): a byte per 64 x 64
+    // block of A, 128 to a 64-row block; blocks whose byte is 0 are not read
+    // (zero: 16 zero bytes stand in).  lo_any (nullable): 0 when all of A2 is
+    // zero.  Neither: A2 is read throughout.
+    const uint8_t *lo_in;
+    const void *zero;
+    const int *lo_any;
+    // GELU split: the flags of the output.  lo_out: a byte per 64 x 64 block, lo
+    // written only where it is 1; lo_any_out: set to 1 where some lo half is
+    // nonzero, lo written throughout.
+    uint8_t *lo_out;
+    int *lo_any_out;
     // f16-pair epilogues (QKV, GELU split): set to 1 when a finite or infinite
     // value reaches |v| >= 65520, where the pair's hi half overflows (nullable)
     int *ovf;
@@ -62,6 +78,7 @@ struct FwGemm {
 
 // false when the operand kind / epilogue pair has no kernel (nothing launched)
 bool fw_launch_gemm(hipStream_t st, int kind, const FwGemm &g);
+bool fw_launch_gemm_f16(hipStream_t st, const FwGemm &g, int ncu); // the f16-pair kind (enc_gemm_f16.hip)
 // ovf (nullable): as FwGemm::ovf, for the SPLIT output.  With FW_LN_SEQ,
 // stats [rows][2] (f64) is scratch for the sequential statistics (required).
 void fw_launch_enc_ln(hipStream_t st, const float *x, const float *w, const float *b, int rows, int d, int mode,
@@ -70,7 +87,7 @@ void fw_launch_enc_ln(hipStream_t st, const float *x, const float *w, const floa
 void fw_launch_quant_exact_rows(hipStream_t st, const float *x, int rows, int n, int8_t *q, float *qs);
 // The f16 copy of the GELU table that follows the f32 one (65536 entries) in
 // the context's allocation; tab is the context's f32 table.
-inline const uint16_t *fw_gelu_tab16(const float *tab) { return (const uint16_t *)(tab + 65536); }
+__host__ __device__ inline const uint16_t *fw_gelu_tab16(const float *tab) { return (const uint16_t *)(tab + 65536); }
 void fw_launch_gelu_quant_i7_rows(hipStream_t st, const float *x, int rows, int n, const float *tab, int8_t *q,
                                   float *qs);
 // The same GELU + quantization from FW_EPI_F16IDX rows (f16 table indices hx,
@@ -78,8 +95,11 @@ void fw_launch_gelu_quant_i7_rows(hipStream_t st, const float *x, int rows, int 
 // supported width (a multiple of 512 up to 8192).
 bool fw_launch_gelu_quant_h16(hipStream_t st, const uint16_t *hx, const float *side, int rows, int n,
                               const float *tab, int8_t *q, float *qs);
-void fw_launch_im2col(hipStream_t st, const float *x, int B, int Tin, int Cin, int stride, int Tout, int Kp,
-                      uint16_t *hi, uint16_t *lo, int *ovf = nullptr);
+// im2col of conv1 (3 taps, stride 1, pad 1) into an f16 pair [B*T, Kp]; also
+// zeroes the padding rows (0 and T + 1) of every window in conv1's output pair
+// oh / ol [B, T + 2, d] and clears *lo_any
+void fw_launch_im2col(hipStream_t st, const float *x, int B, int T, int Cin, int Kp, uint16_t *hi, uint16_t *lo,
+                      int *ovf, uint16_t *oh, uint16_t *ol, int d, int *lo_any);
 void fw_launch_mel_window(hipStream_t st, const float *mel, int n_mel, long long mel_frames, const long long *offs,
                           int n_frames, float *out, int B);
 void fw_launch_fill_u16(hipStream_t st, uint16_t *p, size_t n, uint16_t v);

@@ -1,0 +1,92 @@
+"""The f16-pair GEMMs at the edges of their tiles and of the GELU outputs' lo
+planes: row counts around 64 / 128 / 256, windows that straddle row tiles (the
+conv stem's padded layout), MLP and conv rows with values >= 10 (whose lo
+halves are nonzero) in some 64 x 64 blocks only, and one encoder used with
+other frame counts in between (nothing left over from a larger call).
+
+Fast mode against exact mode (bit-identical to the oracle): pairs carry |a| to
+2^-22 relative with f32 sums, so a GELU argument can round to the neighbouring
+f16 table index and move one fc2 input by 2^-11 of it; bound 1e-3 max-abs, as
+for the whole f32 plan.  With six fc1 values of about 300 a row's maximum is
+about 300 * 0.03 * sqrt(6) = 22 (weights ~0.03): an index step there is at most
+2^-11 * 10 * 0.03 / 22 = 7e-6 and a few together stay under 1e-4, while a lo
+plane that is skipped or stale (2^-12 of 300 per value) would show as 1e-4 ..
+6e-4."""
+import copy
+
+import numpy as np
+import pytest
+
+from franken_whisper_amd import abi, native, synth
+from tests.helpers import assert_bitexact, rel_maxabs
+
+pytestmark = pytest.mark.gpu
+
+CFG = synth.Config("gemm-edges", 51864, 640, 384, 6, 2, 64, 384, 6, 1, 16)
+
+
+def _model(gain):
+    """gain: the factor on a few MLP LayerNorm weights (fc1 values pass 10 in some blocks)."""
+    m = copy.copy(synth.Model(CFG, seed=5, decoder=False))
+    if gain:
+        m.t = dict(m.t)
+        for i in range(CFG.n_audio_layer):
+            name = f"encoder.blocks.{i}.mlp.0.bias"
+            b = m.t[name].copy()
+            b[70:75] += np.float32(gain)  # one 64-column block of fc1 (two with the next at 1000)
+            b[1000] += np.float32(gain)
+            m.t[name] = b
+    return m
+
+
+@pytest.fixture(scope="module")
+def encs():
+    ctx = native.Context(0)
+    made = {}
+
+    def get(plan, gain):
+        if (plan, gain) not in made:
+            made[plan, gain] = native.Encoder(ctx, _model(gain), plan)
+        return ctx, made[plan, gain]
+
+    yield get
+    for e in made.values():
+        e.close()
+    ctx.close()
+
+
+def _forward(ctx, e, x, rows, exact=False):
+    out = ctx.empty((x.shape[0], rows, CFG.n_audio_state), np.float32)
+    e.set_exact(exact)
+    e.forward_time_major(ctx.array(np.ascontiguousarray(x)), x.shape[0], 2 * rows, out)
+    e.set_exact(False)
+    return out.download()
+
+
+@pytest.mark.parametrize("gain", [0, 11, 300], ids=["small", "values-10", "values-300"])
+@pytest.mark.parametrize("rows,n", [(1, 1), (1, 5), (2, 3), (31, 3), (32, 2), (63, 2), (64, 4), (65, 5), (127, 2), (129, 3),
+                                    (255, 2), (257, 3), (300, 40), (513, 2), (640, 8)])
+def test_f32_plan_tile_edges(encs, rows, n, gain):
+    ctx, e = encs(abi.ENC_F32, gain)
+    x = synth.mel_input(rows, n, 2 * rows, CFG.n_mels) * np.float32(0.5)
+    got = _forward(ctx, e, x, rows)
+    want = _forward(ctx, e, x, rows, exact=True)
+    err = rel_maxabs(got, want)
+    print("rows", rows, "windows", n, "gain", gain, "error", err, flush=True)
+    assert err < (1e-4 if gain == 300 else 1e-3)
+
+
+@pytest.mark.parametrize("plan", [abi.ENC_F32, abi.ENC_INT8], ids=["f32", "int8"])
+def test_calls_of_other_sizes_leave_nothing(encs, plan):
+    """Large conv inputs (conv1 outputs >= 10, a nonzero lo plane), then shorter
+    and smaller ones on the same buffers: the same bits as before."""
+    ctx, e = encs(plan, 0)
+    small = [(100, 3), (300, 2), (640, 1)]
+    xs = [synth.mel_input(7 + r, n, 2 * r, CFG.n_mels) * np.float32(0.5) for r, n in small]
+    first = [_forward(ctx, e, x, r) for x, (r, n) in zip(xs, small)]
+    big = synth.mel_input(3, 4, 2 * 640, CFG.n_mels) * np.float32(400.0)
+    got = _forward(ctx, e, big, 640)
+    if plan == abi.ENC_F32:
+        assert rel_maxabs(got, _forward(ctx, e, big, 640, exact=True)) < 1e-3
+    for x, (r, n), want in zip(xs, small, first):
+        assert_bitexact(_forward(ctx, e, x, r), want, f"{r} rows x {n} after larger calls")
