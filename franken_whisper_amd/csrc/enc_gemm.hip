@@ -451,6 +451,14 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
 // for every wave so the counts above stay uniform; a tile's scales sit in the
 // LDS half of its parity).
 //
+// What bounds it: a 256 x 256 stage takes 1,550-1,750 cycles for 1,060 of MFMAs
+// (the stage barrier with both waves of a SIMD at it, LDS at three quarters of
+// its rate), a tile's epilogue 15,000-18,000 against 35,000 for its 20 stages at K
+// 1280 (conversion of the accumulators, store instructions), the clock falls to
+// 1.6-1.9 GHz under it.  With the loads and fragment reads between the MFMAs
+// instead of after the barrier (10 windows): q/k/v 146 -> 127 us, attn.out 66 ->
+// 56, fc1 150 -> 146, fc2 165 -> 155.
+//
 // Tile sequence: XCD x (blocks x, x+8, ...) owns a contiguous range of the
 // GM=8-grouped tile order, walked by its blocks in lockstep, so the tiles in
 // flight on one XCD share A row panels and B column panels in its L2.  With
@@ -458,7 +466,7 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
 // each window is tiled on its own, so every tile's rows share one window and
 // start at a multiple of BM within it.
 template <int EPI, int BM, int BN, int WGM, int WGN, int NS>
-__global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_pi8(FwGemm g, int ntm, int ntn, int ntw) {
+__global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_pi8(FwGemm g, int ntm, int ntn, int ntw) {
     constexpr int NW = WGM * WGN, WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
     constexpr int STAGE = (BM + BN) * 64, LPW = STAGE / 1024 / NW;
     constexpr int SCL = (BM + 2 * BN + 64 * NW - 1) / (64 * NW); // scale loads per wave per tile
@@ -470,7 +478,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_pi8(FwGemm g, int ntm, 
     static_assert(STAGE % (1024 * NW) == 0, "stage loads must split evenly over waves");
     __shared__ __align__(1024) unsigned char lds[NS * STAGE + 2 * SCLN * 4 + NW * SLABB];
     float *scl = (float *)(lds + NS * STAGE);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
     const int G = gridDim.x, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3, nloc = G >> 3;
     const int ntiles = ntm * ntn;
@@ -497,21 +505,23 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_pi8(FwGemm g, int ntm, 
             mrows = min(BM, g.M - m0);
         }
     };
-    // issue side: tile and step of the next stage to load, per-lane sources
+    // issue side: tile and step of the next stage to load; per-lane 32-bit
+    // offsets from the tile's operand panels, per-lane scale sources
     int it_tile = 0, it_step = 0;
-    const unsigned char *src[LPW];
+    const unsigned char *pa, *pb;
+    uint32_t off[LPW];
     const float *ssrc[SCL];
-    auto set_src = [&](int ti) {
+    auto set_src = [&](int ti) __attribute__((always_inline)) {
         int m0, mrows, n0;
         coords(ti, m0, mrows, n0);
+        pa = (const unsigned char *)g.A + (size_t)m0 * g.lda;
+        pb = (const unsigned char *)g.B + (size_t)n0 * g.ldb;
 #pragma unroll
         for (int q = 0; q < LPW; q++) {
             const int lr = (wave * LPW + q) * 16 + (lane >> 2);
             const int c = (lane & 3) ^ gsw(lr);
-            if (lr < BM)
-                src[q] = (const unsigned char *)g.A + (size_t)(m0 + min(lr, mrows - 1)) * g.lda + c * 16;
-            else
-                src[q] = (const unsigned char *)g.B + (size_t)min(n0 + lr - BM, g.N - 1) * g.ldb + c * 16;
+            if (lr < BM) off[q] = (uint32_t)min(lr, mrows - 1) * g.lda + c * 16;
+            else off[q] = (uint32_t)min(lr - BM, g.N - 1 - n0) * g.ldb + c * 16;
         }
 #pragma unroll
         for (int q = 0; q < SCL; q++) {
@@ -522,19 +532,24 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_pi8(FwGemm g, int ntm, 
         }
     };
     set_src(0);
-    auto issue = [&](int gs) {
-        unsigned char *dst = lds + (gs % NS) * STAGE + wave * LPW * 1024;
+    // load q of stage gs
+    auto issue = [&](int gs, int q) __attribute__((always_inline)) {
+        unsigned char *dst = lds + (gs % NS) * STAGE + (wave * LPW + q) * 1024;
         const int sc = it_tile < my_n ? it_step : nsteps - 1; // past the last tile: in-bounds reload
-#pragma unroll
-        for (int q = 0; q < LPW; q++)
-            __builtin_amdgcn_global_load_lds((const void *)(src[q] + (size_t)sc * 64),
-                                             (void __attribute__((address_space(3))) *)(dst + q * 1024), 16, 0, 0);
+        // (a mask, not a choice between the captured pointers, which would keep them in memory)
+        const unsigned long long a = (unsigned long long)pa, b = (unsigned long long)pb;
+        const unsigned long long base = a + (((wave * LPW + q) * 16 < BM ? 0ull : ~0ull) & (b - a)) + (size_t)sc * 64;
+        __builtin_amdgcn_global_load_lds((const void *)((const char *)base + off[q]),
+                                         (void __attribute__((address_space(3))) *)dst, 16, 0, 0);
+    };
+    // after a stage's last load: the scales of a new tile, the next stage
+    auto advance = [&]() __attribute__((always_inline)) {
         if (it_step == 0) {
             float *sd = scl + (it_tile & 1) * SCLN + wave * 64;
 #pragma unroll
-            for (int q = 0; q < SCL; q++)
-                __builtin_amdgcn_global_load_lds((const void *)ssrc[q],
-                                                 (void __attribute__((address_space(3))) *)(sd + q * NW * 64), 4,
+            for (int e = 0; e < SCL; e++)
+                __builtin_amdgcn_global_load_lds((const void *)ssrc[e],
+                                                 (void __attribute__((address_space(3))) *)(sd + e * NW * 64), 4,
                                                  0, 0);
         }
         if (++it_step == nsteps) {
@@ -554,51 +569,68 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_pi8(FwGemm g, int ntm, 
         for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0;
-    v4i fa[2][TM], fb[2][TN];
-    auto ldfrag = [&](int set, int stage, int ks) {
+    // fragment x (A tiles, then B tiles) of substep ks of a stage
+    constexpr int NF = TM + TN, NM = TM * TN, LH = LPW / 2;
+    v4i fr[2][NF];
+    auto ldfrag = [&](int set, int stage, int ks, int x) __attribute__((always_inline)) {
         const unsigned char *tb = lds + (stage % NS) * STAGE;
         const int c = ks * 2 + (lane >> 5);
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-            const int lr = wm * WM + i * 32 + (lane & 31);
-            fa[set][i] = *(const v4i *)(tb + lr * 64 + ((c ^ gsw(lr)) << 4));
-        }
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int lr = BM + wn * WN + j * 32 + (lane & 31);
-            fb[set][j] = *(const v4i *)(tb + lr * 64 + ((c ^ gsw(lr)) << 4));
-        }
+        const int lr = (x < TM ? wm * WM + x * 32 : BM + wn * WN + (x - TM) * 32) + (lane & 31);
+        fr[set][x] = *(const v4i *)(tb + lr * 64 + ((c ^ gsw(lr)) << 4));
     };
-    auto mfmas = [&](int set) {
+    // Half a stage: the MFMAs of one substep with the next substep's fragment
+    // reads and loads [q0, q1) of a later stage between them (requested all at
+    // once after the barrier they hold the wave's MFMAs up).
+    auto half = [&](int set, int rstage, int rks, int lstage, int q0, int q1, bool on) __attribute__((always_inline)) {
+        int rd = 0, ld = q0;
 #pragma unroll
-        for (int i = 0; i < TM; i++)
+        for (int m = 0; m < NM; m++) {
+            const int i = m / TN, j = m % TN;
+            acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fr[set][i], fr[set][TM + j], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < TN; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[set][i], fb[set][j], acc[i][j], 0, 0, 0);
+            for (int u = 0; u < NF; u++)
+                if (rd < NF && (m + 1) * NF * 4 >= (rd + 1) * NM * 3) ldfrag(set ^ 1, rstage, rks, rd++);
+            if (ld < q1 && (m + 1) * (q1 - q0) * 2 >= (ld - q0 + 1) * NM) {
+                if (on) issue(lstage, ld);
+                ld++;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int u = 0; u < LPW; u++)
+            if (ld < q1) {
+                if (on) issue(lstage, ld);
+                ld++;
+            }
     };
 
+#pragma unroll 1
+    for (int p = 0; p < NS - 1; p++) {
 #pragma unroll
-    for (int p = 0; p < NS - 1; p++) issue(p);
+        for (int q = 0; q < LPW; q++) issue(p, q);
+        advance();
+    }
     FW_WAIT_VM(0);
     asm volatile("s_barrier" ::: "memory");
-    issue(NS - 1);
-    ldfrag(0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < LH; q++) issue(NS - 1, q);
+#pragma unroll
+    for (int x = 0; x < NF; x++) ldfrag(0, 0, 0, x);
     const bool has_bias = g.bias != nullptr;
     int tile = 0, s = 0;
     for (int gs = 0; gs < total; gs++) {
-        FW_WAIT_LGKM0();
-        ldfrag(1, gs, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(0);
-        __builtin_amdgcn_sched_barrier(0);
-        FW_WAIT_VM_LGKM0(LPW * (NS - 2));
+        FW_WAIT_LGKM0(); // set 0, read during the last MFMAs
+        half(0, gs, 1, gs + NS - 1, LH, LPW, true);
+        advance();
+        // stage gs+1 visible to every wave.  At a tile's first step it landed
+        // before the last epilogue's stores (or in the prologue), which are
+        // left to drain.
+        if (s == 0) FW_WAIT_LGKM0();
+        else FW_WAIT_VM_LGKM0(LPW * (NS - 2));
         asm volatile("s_barrier" ::: "memory");
         const bool last = s == nsteps - 1;
-        if (!last) issue(gs + NS);
-        ldfrag(0, gs + 1, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        mfmas(1);
-        __builtin_amdgcn_sched_barrier(0);
+        half(1, gs + 1, 0, gs + NS, 0, LH, !last); // (a tile's last step loads after its stores)
         if (!last) {
             s++;
             continue;
@@ -790,7 +822,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN) k_gemm_pi8(FwGemm g, int ntm, 
             for (int j = 0; j < TN; j++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[i][j][r] = 0;
-        issue(gs + NS);
+#pragma unroll
+        for (int q = 0; q < LH; q++) issue(gs + NS, q);
         tile++;
         s = 0;
     }
@@ -858,13 +891,17 @@ static void launch_tiles(hipStream_t st, const FwGemm &g, int tile) {
     }
 }
 
-// Persistent int8 launch: 256x256 tiles (8 waves of 128x64) for wide outputs,
-// 256x128 (8 waves of 64x64) for N < 2048 and for the residual epilogue, whose
-// wave tile must fit its residual values in registers.  One block per CU
-// (LDS and registers admit no second); the grid is a multiple of 8 so block
-// b runs on XCD b % 8.
-template <int EPI, int BM, int BN, int WGM, int WGN>
-static void launch_pi8(hipStream_t st, const FwGemm &g, int ncu) {
+// Persistent int8 launch.  256x256 tiles (8 waves of 128x64) or 256x128 (8 of
+// 64x64), one block per CU, or 128x128 (4 of 64x64), two; the residual epilogue,
+// whose wave tile must fit its residual values in registers, takes the latter
+// two.  The grid is a multiple of 8 so block b runs on XCD b % 8.
+//
+// The choice is the fewest rounds of the CUs, weighted by a round's time
+// relative to 256x256 (measured, K 1280, 10 windows: 27 us, 15 for 256x128, 16
+// for two 128x128 a CU, less where one a CU suffices: one and two windows' fc2
+// 47 -> 39 us).
+template <int EPI, int BM, int BN, int WGM, int WGN, int NS>
+static void launch_pi8(hipStream_t st, const FwGemm &g, int ncu, int per_cu) {
     int ntw = 0, ntm;
     if (EPI == FW_EPI_QKV) {
         ntw = (g.T + BM - 1) / BM;
@@ -874,18 +911,27 @@ static void launch_pi8(hipStream_t st, const FwGemm &g, int ncu) {
     }
     const int ntn = (g.N + BN - 1) / BN;
     const int grid = ncu >= 8 ? ncu / 8 * 8 : 8;
-    hipLaunchKernelGGL((k_gemm_pi8<EPI, BM, BN, WGM, WGN, 3>), dim3(grid), dim3(64 * WGM * WGN), 0, st, g, ntm, ntn,
-                       ntw);
+    hipLaunchKernelGGL((k_gemm_pi8<EPI, BM, BN, WGM, WGN, NS>), dim3(grid * per_cu), dim3(64 * WGM * WGN), 0, st, g,
+                       ntm, ntn, ntw);
 }
 
 template <int EPI>
 static void launch_pi8_tiles(hipStream_t st, const FwGemm &g, int ncu) {
+    auto blocks = [&](int bm, int bn) {
+        const long long tm = EPI == FW_EPI_QKV ? (long long)(g.M / g.T) * ((g.T + bm - 1) / bm) : (g.M + bm - 1) / bm;
+        return tm * ((g.N + bn - 1) / bn);
+    };
+    const long long n2 = blocks(128, 128), left = n2 % (2 * ncu);
+    const double c0 = (double)((blocks(256, 256) + ncu - 1) / ncu);
+    const double c1 = (double)((blocks(256, 128) + ncu - 1) / ncu) * 0.56;
+    const double c2 = (double)(n2 / (2 * ncu)) * 0.6 + (left == 0 ? 0.0 : left <= ncu ? 0.42 : 0.6);
     if constexpr (EPI != FW_EPI_RESID)
-        if (g.N >= 2048) {
-            launch_pi8<EPI, 256, 256, 2, 4>(st, g, ncu);
+        if (c0 <= c1 && c0 <= c2) {
+            launch_pi8<EPI, 256, 256, 2, 4, 3>(st, g, ncu, 1);
             return;
         }
-    launch_pi8<EPI, 256, 128, 4, 2>(st, g, ncu);
+    if (c1 <= c2) launch_pi8<EPI, 256, 128, 4, 2, 3>(st, g, ncu, 1);
+    else launch_pi8<EPI, 128, 128, 2, 2, EPI == FW_EPI_QKV || EPI == FW_EPI_F16IDX ? 3 : 4>(st, g, ncu, 2);
 }
 
 bool fw_launch_gemm(hipStream_t st, int kind, const FwGemm &g0) {
@@ -909,12 +955,7 @@ bool fw_launch_gemm(hipStream_t st, int kind, const FwGemm &g0) {
         pi8 = e ? atoi(e) : 1;
     }
     if (kind == FW_KIND_F16S) return fw_launch_gemm_f16(st, g0, ncu);
-    // One window (M <= 1536 rows) fills the CUs better with the one-tile-per-
-    // block kernels' tiles: the persistent kernel's 256 x 256 tiles give the
-    // q/k/v GEMM 90 tiles for 256 CUs (one-window encoder pass 8.35 -> 7.78
-    // ms; from two windows on the persistent kernel is faster: 9.81 against
-    // 10.15 ms, ten 36.1 against 40.3).  Both routes give the same bits.
-    if (pi8 && g.M > 1536 && g.K % 64 == 0 &&
+    if (pi8 && g.K % 64 == 0 &&
         (g.epi != FW_EPI_QKV || (g.T > 0 && g.M % g.T == 0))) {
         switch (g.epi) {
         case FW_EPI_F32: launch_pi8_tiles<FW_EPI_F32>(st, g, ncu); return true;

@@ -1,0 +1,83 @@
+"""The int8 encoder GEMMs at the edges of their tiles (256 x 256, 256 x 128, 128 x
+128 and where the choice between them changes): the exact accumulators and
+every epilogue against the oracle bit for bit, the fused q/k/v split against the
+f16 pairs of the oracle's values."""
+import numpy as np
+import pytest
+
+from franken_whisper_amd import abi, native, synth
+from oracle import oracle as O
+from tests.helpers import assert_bitexact
+
+pytestmark = pytest.mark.gpu
+
+CFG = synth.Config("i8-edges", 51864, 1500, 384, 6, 1, 64, 384, 6, 1, 16)
+
+
+@pytest.fixture(scope="module")
+def pair():
+    ctx = native.Context(0)
+    m = synth.Model(CFG, seed=9, decoder=False)
+    e = native.Encoder(ctx, m, abi.ENC_INT8)
+    yield ctx, e, O.Encoder(m, abi.ENC_INT8)
+    e.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("M", [1, 31, 32, 33, 127, 128, 129, 255, 256, 257, 700, 1500, 3000, 6001])
+def test_gemm_rows(pair, M):
+    ctx, e, oenc = pair
+    d = CFG.n_audio_state
+    rng = np.random.default_rng(M)
+    for which in (0, 3, 4, 5):
+        inp, out = (4 * d if which == 5 else d), (4 * d if which == 4 else d)
+        x = (rng.standard_normal((M, inp)) * 1.3).astype(np.float32)
+        acc, y = ctx.empty((M, out), np.int32), ctx.empty((M, out), np.float32)
+        print("rows", M, "gemm", which, flush=True)
+        e.gemm_i8(0, which, ctx.array(x), acc, y)
+        want_acc, want_y = oenc.gemm(0, which, x)
+        np.testing.assert_array_equal(acc.download(), want_acc)
+        assert_bitexact(y.download(), want_y, f"rows {M} gemm {which}")
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (3, 31), (2, 64), (1, 129), (5, 255), (2, 257), (1, 1500), (30, 300)])
+def test_qkv_windows(pair, B, T):
+    ctx, e, oenc = pair
+    d, H, Tp = CFG.n_audio_state, CFG.n_audio_head, (T + 63) // 64 * 64
+    x = (np.random.default_rng(T).standard_normal((B * T, d)) * 1.3).astype(np.float32)
+    qk, vt = B * H * T * 64, B * H * 64 * Tp
+    out = ctx.empty((4 * qk + 2 * vt,), np.uint16)
+    print("windows", B, "rows", T, flush=True)
+    e.gemm_i8_fused(0, 0, ctx.array(x), B, T, out)
+    got = out.download()
+    t = np.arange(T)
+    pos = (t & ~12) | ((t & 4) << 1) | ((t & 8) >> 1)
+    for which in range(3):
+        y = np.asarray(oenc.gemm(0, which, x)[1], np.float32)
+        hi = y.astype(np.float16)
+        lo = (y - hi.astype(np.float32)).astype(np.float16)
+        for k, p in enumerate((hi, lo)):
+            want = p.view(np.uint16).reshape(B, T, H, 64)
+            if which < 2:
+                plane = got[(2 * which + k) * qk:(2 * which + k + 1) * qk].reshape(B, H, T, 64)
+                np.testing.assert_array_equal(plane, want.transpose(0, 2, 1, 3))
+            else:
+                plane = got[4 * qk + k * vt:4 * qk + (k + 1) * vt].reshape(B, H, 64, Tp)
+                np.testing.assert_array_equal(plane[:, :, :, pos], want.transpose(0, 2, 3, 1))
+
+
+@pytest.mark.parametrize("M", [1, 33, 129, 257, 1500, 6001])
+def test_fc1_index(pair, M):
+    ctx, e, oenc = pair
+    d = CFG.n_audio_state
+    x = (np.random.default_rng(M).standard_normal((M, d)) * 1.3).astype(np.float32)
+    x[::5] *= 60.0  # rows whose fc1 values pass +-10
+    idx, side = ctx.empty((M, 4 * d), np.uint16), ctx.empty((M, 4 * d), np.float32)
+    print("fc1 index rows", M, flush=True)
+    e.gemm_i8_fused(0, 4, ctx.array(x), 1, M, idx, side)
+    y = oenc.gemm(0, 4, x)[1]
+    inside = np.abs(y) < np.float32(9.98)
+    gi = idx.download()
+    np.testing.assert_array_equal(gi[inside], y[inside].astype(np.float16).view(np.uint16))
+    assert np.all(gi[~inside] == 0xFFFF)
+    assert_bitexact(side.download()[~inside], y[~inside], "fc1 side values")
