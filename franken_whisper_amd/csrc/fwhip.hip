@@ -313,7 +313,7 @@ struct fwhip_dstate {
     int32_t *poll_host = nullptr;
     int poll_cap = 0;
     // batched prompt prefill (f16 arm): activation rows of a chunk of
-    // PF_CHUNK positions x S streams, allocated on first use
+    // pf_chunk(S) positions x S streams, allocated on first use
     std::vector<void *> pf_owned;
     float *pf_x = nullptr, *pf_h = nullptr, *pf_qkv = nullptr, *pf_att = nullptr, *pf_y = nullptr, *pf_ff = nullptr;
     FwWinPart *w_part = nullptr; // [S][WIN_NB] partial results of the select blocks
@@ -994,14 +994,16 @@ static void dec_logits_f16(fwhip_dstate *st, const float *x, float *h, const fwh
     }
 }
 
-// Batched prompt prefill (f16 arm): the rows of PF_CHUNK positions of every
+// Batched prompt prefill (f16 arm): the rows of pf_chunk(S) positions of every
 // stream go through each layer together, [position][stream] order, row r at
 // stream r % S and position *pos + r / S.  Every projection is row-local
 // (gemv_f16 per row), so a batch gives each row the bits of its own forward;
 // the self attention appends every row's k/v first and then lets row r see
 // positions [0, *pos + r / S] of its stream, exactly the keys the row-by-row
 // forward gives it (decoder.rs:1754-1906).
-#define PF_CHUNK 32
+// A chunk is 32 positions, more while its rows stay within 256: the GEMMs'
+// 16-row tiles then fill the chip (one stream's 227 rows: 8 chunks of 32 before).
+static int pf_chunk(int S) { return S >= 8 ? 32 : 256 / S; }
 static bool prefill_batch_ok(const fwhip_dstate *st) {
     const fwhip_decoder *dd = st->dec;
     return dd->arm == FWHIP_DEC_F16 && st->ck16p && fw_cross_f16p_ok(st->T) && dd->d == dd->H * 64 &&
@@ -1011,7 +1013,7 @@ static bool prefill_batch_ok(const fwhip_dstate *st) {
 static fwhip_status prefill_buffers(fwhip_dstate *st) {
     if (st->pf_x) return FWHIP_OK;
     const fwhip_decoder *dd = st->dec;
-    const size_t R = (size_t)st->S * PF_CHUNK, d = dd->d;
+    const size_t R = (size_t)st->S * pf_chunk(st->S), d = dd->d;
     st->pf_x = (float *)fw_dalloc(st->pf_owned, sizeof(float) * R * d);
     st->pf_h = (float *)fw_dalloc(st->pf_owned, sizeof(float) * R * dd->dff);
     st->pf_qkv = (float *)fw_dalloc(st->pf_owned, sizeof(float) * R * 3 * d);
@@ -1090,8 +1092,9 @@ static fwhip_status stage_rows(fwhip_dstate *st, const int32_t *tokens, int tq, 
     if (tq > 1 && prefill_batch_ok(st)) {
         r = prefill_buffers(st);
         if (r != FWHIP_OK) return r;
-        for (int c0 = 0; c0 < tq; c0 += PF_CHUNK) {
-            const int n = tq - c0 < PF_CHUNK ? tq - c0 : PF_CHUNK, p = p0 + c0;
+        const int ch = pf_chunk(S);
+        for (int c0 = 0; c0 < tq; c0 += ch) {
+            const int n = tq - c0 < ch ? tq - c0 : ch, p = p0 + c0;
             r = set_dev_ints(c, st->pos, &p, 1);
             if (r != FWHIP_OK) return r;
             r = dec_forward_chunk(st, st->rows + (size_t)c0 * S, n, c0 + n == tq, filt, true);
