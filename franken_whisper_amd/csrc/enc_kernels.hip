@@ -597,6 +597,28 @@ __device__ __forceinline__ float at_sum32(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+// one query's output row: dims t*32 + q*8 + (lane/32)*4 .. +3
+__device__ __forceinline__ void at_store(const v16f (&o)[2], float inv, size_t orow, int lane, int out_mode, float *of,
+                                         uint16_t *oh, uint16_t *ol) {
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const size_t oo = orow + t * 32 + q * 8 + (lane >> 5) * 4;
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = o[t][q * 4 + e] * inv;
+            if (out_mode == 0) {
+                *(float4 *)(of + oo) = make_float4(v[0], v[1], v[2], v[3]);
+            } else {
+                uint16_t hi[4], lw[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) fw_split(v[e], hi[e], lw[e]);
+                *(uint2 *)(oh + oo) = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
+                *(uint2 *)(ol + oo) = make_uint2(lw[0] | ((uint32_t)lw[1] << 16), lw[2] | ((uint32_t)lw[3] << 16));
+            }
+        }
+}
 template <int QPW>
 __global__ void __launch_bounds__(512, 2) k_attention3(const uint16_t *qh, const uint16_t *ql, const uint16_t *kh,
                                                        const uint16_t *kl, const uint16_t *vth, const uint16_t *vtl,
@@ -836,29 +858,196 @@ __global__ void __launch_bounds__(512, 2) k_attention3(const uint16_t *qh, const
         if (myq >= T) continue;
         const float inv = 1.0f / l[qs];
         const size_t orow = ((size_t)b * T + myq) * d + (size_t)h * 64;
-        // dims t*32 + q*8 + (lane/32)*4 .. +3 of the row
-        if (out_mode == 0) {
+        at_store(o[qs], inv, orow, lane, out_mode, of, oh, ol);
+    }
+}
+
+// The same for few blocks (a window or two): 128 queries per block of 4 waves,
+// each wave overlapping by itself.  Iteration j multiplies P V of tile j - 1 and
+// the scores of tile j + 1 while it exponentiates tile j: the exps of four scores
+// a lane lie between every six MFMAs.  Slot j % 2 of the ring holds the K of tile
+// j + 1 and the V of tile j - 1.  Per query the operations of k_attention3 in the
+// same order.
+__global__ void __launch_bounds__(256, 2) k_attention_few(const uint16_t *qh, const uint16_t *ql, const uint16_t *kh,
+                                                          const uint16_t *kl, const uint16_t *vth,
+                                                          const uint16_t *vtl, int T, int Tp, int H, int d, int nq,
+                                                          int out_mode, float *of, uint16_t *oh, uint16_t *ol) {
+    __shared__ __align__(1024) uint16_t sm[2][4][AT_TILE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nb = gridDim.x, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3, per = nb >> 3, rem = nb & 7;
+    const int bt = xcd < rem ? xcd * (per + 1) + loc : rem * (per + 1) + (xcd - rem) * per + loc;
+    const size_t bh = bt / nq;
+    const int b = (int)(bh / H), h = (int)(bh - (size_t)b * H);
+    const int myq = ((bt - (int)bh * nq) * 4 + wave) * 32 + (lane & 31), qc = myq < T ? myq : T - 1;
+    const int nt = (T + 63) >> 6;
+    v8h qfh[4], qfl[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) {
+        const size_t o = (bh * T + qc) * 64 + ks * 16 + (lane >> 5) * 8;
+        qfh[ks] = *(const v8h *)(qh + o);
+        qfl[ks] = *(const v8h *)(ql + o);
+    }
+    // loader: wave w loads array w of a pair, 8 instructions of 8 rows
+    const int lr = lane >> 3, lc = ((lane & 7) ^ lr) * 8;
+    const uint32_t lstep = wave < 2 ? 64 : Tp, loff = (lr * lstep + lc) * 2;
+    const char *src = (const char *)(wave == 0 ? kh + bh * T * 64 : wave == 1 ? kl + bh * T * 64
+                                     : wave == 2 ? vth + bh * 64 * Tp : vtl + bh * 64 * Tp);
+    auto issue = [&](int j) {
+        const int tile = wave < 2 ? j + 1 : j - 1;
+        if (tile < 0 || tile >= nt) return;
+        uint16_t *base = &sm[j & 1][wave][0];
+        const int k0 = tile * 64;
+        if (wave < 2 && k0 + 64 > T) {
+            // the last tile's key rows past T reload row T - 1 (masked in the softmax)
+#pragma unroll 1
+            for (int q = 0; q < 8; q++)
+                __builtin_amdgcn_global_load_lds((const void *)(src + (min(k0 + q * 8 + lr, T - 1) * 64 + lc) * 2),
+                                                 (void __attribute__((address_space(3))) *)(base + q * 512), 16, 0, 0);
+            return;
+        }
+        const char *p = src + (size_t)(wave < 2 ? k0 * 64 : k0) * 2;
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+            __builtin_amdgcn_global_load_lds((const void *)(p + (size_t)(q * 16 * lstep) + loff),
+                                             (void __attribute__((address_space(3))) *)(base + q * 512), 16, 0, 0);
+    };
+    const float sl2 = 0.125f * 1.4426950408889634f;
+    const v16f zero = {};
+    v16f o[2] = {zero, zero}, st[2], sn[2];
+    uint32_t ph[2][8], pl[2][8], nh[2][8], nl[2][8];
+    float m = -INFINITY, l = 0.0f;
+    const int fr = lane & 31, fx = lane & 7, fh = lane >> 5;
+    auto frag = [&](const uint16_t *a, int s, v8h (&f)[4]) {
+        const int off = fr * 64 + (((s * 2 + fh) ^ fx) << 3);
+        f[0] = *(const v8h *)(a + off);
+        f[1] = *(const v8h *)(a + 32 * 64 + off);
+        f[2] = *(const v8h *)(a + AT_TILE + off);
+        f[3] = *(const v8h *)(a + AT_TILE + 32 * 64 + off);
+    };
+    // steps 0-3: O += V P of the 16-key group s; steps 4-7: scores over 16 dims
+    auto body = [&](int j, auto hasv, auto hask, auto soft) {
+        constexpr bool HV = decltype(hasv)::value, HK = decltype(hask)::value, SM = decltype(soft)::value;
+        constexpr int S0 = HV ? 0 : 4, S1 = HK ? 8 : 4;
+        const uint16_t *sl = &sm[j & 1][0][0];
+        v8h f[2][4];
+        auto rd = [&](int s) { frag(sl + (s < 4 ? 2 * AT_TILE : 0), s & 3, f[s & 1]); };
+        if (S0 < S1) rd(S0);
+        float mnew = m, nms = 0.0f, psum = 0.0f;
+        if constexpr (SM) {
+            const int k0 = j * 64;
+            if (k0 + 64 > T) {
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const int key = k0 + t * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+                        if (key >= T) st[t][r] = -INFINITY;
+                    }
+            }
+            float tmax = -INFINITY;
 #pragma unroll
             for (int t = 0; t < 2; t++)
 #pragma unroll
-                for (int q = 0; q < 4; q++)
-                    *(float4 *)(of + orow + t * 32 + q * 8 + (lane >> 5) * 4) =
-                        make_float4(o[qs][t][q * 4] * inv, o[qs][t][q * 4 + 1] * inv, o[qs][t][q * 4 + 2] * inv,
-                                    o[qs][t][q * 4 + 3] * inv);
-        } else {
+                for (int r = 0; r < 16; r++) tmax = fmaxf(tmax, st[t][r]);
+            mnew = fmaxf(m, at_max32(tmax));
+            nms = -mnew * sl2;
+        }
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const bool mm = s >= S0 && s < S1;
+            if (mm) {
+                FW_WAIT_LGKM0();
+                if (s + 1 < S1) rd(s + 1);
+            }
+            v8h bhi, blo;
+            if (s < 4) {
+                bhi = __builtin_bit_cast(v8h, make_uint4(ph[s >> 1][(s & 1) * 4], ph[s >> 1][(s & 1) * 4 + 1],
+                                                         ph[s >> 1][(s & 1) * 4 + 2], ph[s >> 1][(s & 1) * 4 + 3]));
+                blo = __builtin_bit_cast(v8h, make_uint4(pl[s >> 1][(s & 1) * 4], pl[s >> 1][(s & 1) * 4 + 1],
+                                                         pl[s >> 1][(s & 1) * 4 + 2], pl[s >> 1][(s & 1) * 4 + 3]));
+            } else {
+                bhi = qfh[s - 4];
+                blo = qfl[s - 4];
+                if (s == 4 && HK) sn[0] = sn[1] = zero;
+            }
+            v16f *acc = s < 4 ? o : sn;
+            auto two = [&](int q) {
+                if (!mm) return;
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f[s & 1][(q == 1 ? 2 : 0) + t], q == 2 ? blo : bhi,
+                                                                    acc[t], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            const int t = s >> 2, r = (s & 3) * 4;
+            float e[4];
+            two(0);
+            if constexpr (SM) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) e[u] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[t][r + u], sl2, nms));
+            }
+            two(1);
+            if constexpr (SM) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) psum += e[u];
+                at_split4(e, nh[t][r >> 1], nh[t][(r >> 1) + 1], nl[t][r >> 1], nl[t][(r >> 1) + 1]);
+            }
+            two(2);
+        }
+        if constexpr (SM) {
+            if (__builtin_amdgcn_ballot_w64(mnew != m)) {
+                const float alpha = __builtin_amdgcn_exp2f((m - mnew) * sl2);
+                l *= alpha;
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) o[t][r] *= alpha;
+            }
+            l += at_sum32(psum);
+            m = mnew;
 #pragma unroll
             for (int t = 0; t < 2; t++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    uint16_t hi[4], lw[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) fw_split(o[qs][t][q * 4 + e] * inv, hi[e], lw[e]);
-                    const size_t oo = orow + t * 32 + q * 8 + (lane >> 5) * 4;
-                    *(uint2 *)(oh + oo) = make_uint2(hi[0] | ((uint32_t)hi[1] << 16), hi[2] | ((uint32_t)hi[3] << 16));
-                    *(uint2 *)(ol + oo) = make_uint2(lw[0] | ((uint32_t)lw[1] << 16), lw[2] | ((uint32_t)lw[3] << 16));
+                for (int r = 0; r < 8; r++) {
+                    ph[t][r] = nh[t][r];
+                    pl[t][r] = nl[t][r];
                 }
         }
+        if constexpr (HK) {
+            st[0] = sn[0];
+            st[1] = sn[1];
+        }
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    auto next = [&](int j) { // pair j has landed everywhere, the slot of pair j - 1 is free
+        FW_WAIT_VM_LGKM0(0);
+        asm volatile("s_barrier" ::: "memory");
+        issue(j + 1);
+    };
+    issue(-1);
+    next(-1);
+    body(-1, no, yes, no); // the scores of tile 0
+    if (nt == 1) {
+        next(0);
+        body(0, no, no, yes);
+    } else {
+        next(0);
+        body(0, no, yes, yes);
+        for (int j = 1; j + 1 < nt; j++) {
+            next(j);
+            body(j, yes, yes, yes);
+        }
+        next(nt - 1);
+        body(nt - 1, yes, no, yes);
     }
+    next(nt);
+    body(nt, yes, no, no);
+    if (myq >= T) return;
+    const float inv = 1.0f / l;
+    const size_t orow = ((size_t)b * T + myq) * d + (size_t)h * 64;
+    at_store(o, inv, orow, lane, out_mode, of, oh, ol);
 }
 
 // ---------------------------------------------------------------------------
@@ -1215,11 +1404,13 @@ void fw_launch_fill_u16(hipStream_t st, uint16_t *p, size_t n, uint16_t v) {
 void fw_launch_attention(hipStream_t st, const uint16_t *qh, const uint16_t *ql, const uint16_t *kh,
                          const uint16_t *kl, const uint16_t *vth, const uint16_t *vtl, int B, int T, int Tp, int H,
                          int d, int out_mode, float *of, uint16_t *oh, uint16_t *ol) {
-    // Rounds of the CUs (one block each) times the work of a block, which grows
-    // with QPW: 256 or 512 queries per block, the larger one where the smaller
-    // gains nothing (it reads the fragments once per two sub-tiles: 16 windows
-    // 490 us against 537; 10 windows, 3 rounds against 5 half ones, 351 against
-    // 342; two windows 108 against 75).
+    // Up to one round of 128-query blocks: the 4-wave kernel (one window of 20
+    // heads, 240 blocks: 45 us against 59 for 120 blocks of 256; two windows 75
+    // against 71).  Then rounds of the CUs (one block each) times the work of a
+    // block, which grows with QPW: 256 or 512 queries per block, the larger one
+    // where the smaller gains nothing (it reads the fragments once per two
+    // sub-tiles: 16 windows 490 us against 537; 10 windows, 3 rounds against 5
+    // half ones, 351 against 342; two windows 108 against 75).
     static int n_cu = 0;
     if (!n_cu) {
         int dev = 0;
@@ -1232,7 +1423,11 @@ void fw_launch_attention(hipStream_t st, const uint16_t *qh, const uint16_t *ql,
 #define AT_GO(QPW_, NQ_)                                                                                             \
     hipLaunchKernelGGL(k_attention3<QPW_>, dim3((unsigned)(bh * NQ_)), dim3(512), 0, st, qh, ql, kh, kl, vth, vtl, T, \
                        Tp, H, d, NQ_, out_mode, of, oh, ol)
-    if (r1 < r2) AT_GO(1, n1);
+    const int n0 = (T + 127) / 128;
+    if (bh * n0 <= n_cu)
+        hipLaunchKernelGGL(k_attention_few, dim3((unsigned)(bh * n0)), dim3(256), 0, st, qh, ql, kh, kl, vth, vtl, T, Tp,
+                           H, d, n0, out_mode, of, oh, ol);
+    else if (r1 < r2) AT_GO(1, n1);
     else AT_GO(2, n2);
 #undef AT_GO
 }

@@ -1,7 +1,8 @@
 """The f16-pair attention at the edges of its tiles: one 64-key tile, a last
 tile of 1 or 63 keys, query blocks (256 and 512) that end inside a wave or
-leave whole waves without a query.  One window takes the 256-query blocks, 40
-windows the 512-query ones.
+leave whole waves without a query.  One and two windows take the 128-query
+blocks, 7 and more the 256-query ones, 40 windows of 257 to 512 rows the
+512-query ones.
 
 Fast mode against exact mode (bit-identical to the oracle): the pairs carry
 |a| to 2^-22 relative and every sum stays in f32, so the bound is the fast
@@ -35,7 +36,7 @@ def _forward(ctx, e, x, rows):
 @pytest.mark.parametrize("rows", [1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 320, 511, 512, 513, 640])
 def test_attention_tile_edges(enc, rows):
     ctx, e = enc
-    n = 40 if 256 < rows <= 512 else 2  # 240 heads x 2 blocks of 256 queries or 1 of 512
+    n = 40 if 256 < rows <= 512 else 2 if rows < 256 else 15  # 240 heads x 2 blocks of 256 queries or 1 of 512
     x = synth.mel_input(rows, n, 2 * rows, CFG.n_mels) * np.float32(0.5)
     print("rows", rows, "windows", n, flush=True)
     many = _forward(ctx, e, x, rows)
@@ -46,3 +47,7 @@ def test_attention_tile_edges(enc, rows):
     for w in (0, n - 1):
         one = _forward(ctx, e, x[w:w + 1], rows)
         assert_bitexact(one[0], many[w], f"{rows} rows: window {w} alone and among {n}")
+    if rows < 256:  # 43 windows: 258 heads, past one round of 128-query blocks
+        x = np.concatenate([x[:1]] * 43)
+        for y in _forward(ctx, e, x, rows)[::14]:
+            assert_bitexact(y, many[0], f"{rows} rows: among 43 windows")
