@@ -889,7 +889,6 @@ void fw_launch_cross_attn_f16(hipStream_t st, const float *qc, const uint16_t *c
 // 24 rounds of 64 keys) and its V^T groups after its scores; every request is
 // a whole 128-byte line.
 #define XP_MAXG 24 // full 64-key groups of V^T a lane holds in registers
-__device__ __forceinline__ int fw_xp_pos(int e) { return (e & 7) * 8 + (e >> 5) * 4 + ((e >> 3) & 3); }
 
 // FQ: the cross LayerNorm and this head's q rows are formed in the block
 // (gemv_f16 of LN(x_s), nn.rs:2346-2460, on the slot-order matrix of
@@ -1470,22 +1469,42 @@ void fw_launch_cross_attn_f16p_split(hipStream_t st, const float *qc, const uint
 }
 
 // K [rows_k, 64] and V^T [rows_v, T] (natural order) to the slot order of
-// k_cross_attn_f16p; V^T rows take stride Tv (pad left as it is).
+// k_cross_attn_f16p; V^T rows take stride Tv (pad left as it is).  A thread
+// gathers the 8 elements 32 cc + 8 k + l of a 64-wide group that lie together
+// in slot order and stores them at once; blocks below kblk take K, the others a
+// V^T row at a time.  (Bound by HBM and the gathers' 2-byte reads; an element a
+// thread, with a division for its V^T row, took 266 us for ten turbo streams.)
 __global__ void __launch_bounds__(256) k_pack_cross_f16(const uint16_t *ck, const uint16_t *cvt, uint16_t *ckp,
-                                                        uint16_t *cvtp, size_t rows_k, size_t rows_v, int T, int Tv) {
-    const size_t nk = rows_k * 64, nv = rows_v * (size_t)T;
+                                                        uint16_t *cvtp, size_t rows_k, size_t rows_v, int T, int Tv,
+                                                        int kblk) {
+    auto gather = [](const uint16_t *g, int l) {
+        uint16_t u[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) u[q] = g[(q >> 2) * 32 + (q & 3) * 8 + l];
+        return make_uint4(u[0] | ((uint32_t)u[1] << 16), u[2] | ((uint32_t)u[3] << 16), u[4] | ((uint32_t)u[5] << 16),
+                          u[6] | ((uint32_t)u[7] << 16));
+    };
+    if ((int)blockIdx.x < kblk) {
+        for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < rows_k * 8; i += (size_t)kblk * 256)
+            *(uint4 *)(ckp + i * 8) = gather(ck + (i & ~(size_t)7) * 8, (int)(i & 7));
+        return;
+    }
     const int nc = T >> 5, ng = nc >> 1;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < nk + nv; i += (size_t)gridDim.x * 256) {
-        if (i < nk) {
-            ckp[(i & ~(size_t)63) + fw_xp_pos((int)(i & 63))] = ck[i];
-        } else {
-            const size_t iv = i - nk, r = iv / T;
-            const int e = (int)(iv - r * T);
-            int pos;
-            if (e < ng * 64) pos = (e & ~63) + fw_xp_pos(e & 63);
-            else if (e < nc * 32) pos = ng * 64 + ((e - ng * 64) & 7) * 4 + ((e - ng * 64) >> 3);
-            else pos = e;
-            cvtp[r * Tv + pos] = cvt[iv];
+    const int u1 = ng * 8, u2 = u1 + (nc & 1) * 8, units = u2 + (T - nc * 32); // groups, an odd last chunk, the tail
+    for (size_t r = blockIdx.x - kblk; r < rows_v; r += gridDim.x - kblk) {
+        const uint16_t *src = cvt + r * (size_t)T;
+        uint16_t *dst = cvtp + r * (size_t)Tv;
+        for (int u = threadIdx.x; u < units; u += 256) {
+            if (u < u1) {
+                *(uint4 *)(dst + u * 8) = gather(src + (u >> 3) * 64, u & 7);
+            } else if (u < u2) {
+                const int l = u - u1;
+#pragma unroll
+                for (int k = 0; k < 4; k++) dst[ng * 64 + l * 4 + k] = src[ng * 64 + k * 8 + l];
+            } else {
+                const int e = nc * 32 + u - u2;
+                dst[e] = src[e];
+            }
         }
     }
 }
@@ -1497,11 +1516,10 @@ int fw_cross_f16p_tv(int T) { return (T + 63) & ~63; }
 
 void fw_launch_pack_cross_f16(hipStream_t st, const uint16_t *ck, const uint16_t *cvt, uint16_t *ckp, uint16_t *cvtp,
                               size_t rows_k, size_t rows_v, int T) {
-    const size_t tot = rows_k * 64 + rows_v * (size_t)T;
-    size_t g = (tot + 255) / 256;
-    g = g < 65536 ? g : 65536;
-    hipLaunchKernelGGL(k_pack_cross_f16, dim3((unsigned)g), dim3(256), 0, st, ck, cvt, ckp, cvtp, rows_k, rows_v, T,
-                       fw_cross_f16p_tv(T));
+    const size_t kb = (rows_k * 8 + 255) / 256;
+    const int kblk = (int)(kb < 8192 ? kb : 8192), vblk = (int)(rows_v < 8192 ? rows_v : 8192);
+    hipLaunchKernelGGL(k_pack_cross_f16, dim3((unsigned)(kblk + vblk)), dim3(256), 0, st, ck, cvt, ckp, cvtp, rows_k,
+                       rows_v, T, fw_cross_f16p_tv(T), kblk);
 }
 
 void fw_launch_cross_attn_f16p(hipStream_t st, const float *qc, const uint16_t *ckp, const uint16_t *cvtp, float *att,
