@@ -41,9 +41,9 @@ def _classes():
     # kernel class -> (name, roofline bound, MFMA operand type, traffic record)
     return {
         abi.K_ENC_GEMM_I8: ("encoder int8 GEMM (k_gemm_pi8, persistent int8 tiles)", "mfma", "int8", "enc_gemm_i8"),
-        abi.K_ENC_GEMM_F32: ("encoder f16-pair GEMM (k_gemm2, conv stem)", "mfma", "f16", None),
-        abi.K_ENC_ATTN: ("encoder attention (k_attention2, f16 pairs)", "mfma", "f16", None),
-        abi.K_DEC_CROSS: ("decoder cross K/V precompute (k_gemm2 f16 pairs, all layers)", "mfma", "f16", None),
+        abi.K_ENC_GEMM_F32: ("encoder f16-pair GEMM (k_gemm_f16, conv stem)", "mfma", "f16", None),
+        abi.K_ENC_ATTN: ("encoder attention (k_attention3, f16 pairs)", "mfma", "f16", None),
+        abi.K_DEC_CROSS: ("decoder cross K/V precompute (k_gemm_f16 f16 pairs, all layers)", "mfma", "f16", None),
         abi.K_DEC_STEP: ("decoder step (graph replay of one sampled step: weights + cross K/V + KV cache)",
                          "hbm", None, "dec_step"),
         abi.K_DEC_LOGITS: ("decoder logits GEMV of the prompt row (k_gemv_i8m)", "hbm", None, None),

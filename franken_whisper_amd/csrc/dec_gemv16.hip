@@ -431,10 +431,10 @@ void fw_launch_gemv16(hipStream_t st, const uint16_t *Wp, const float *bias, con
     G16Args a{Wp, bias, x, y, N, K, ns, ldy, mode, gelu_tab, lnw, lnb, {}, filt != nullptr, initialp, keys};
     if (filt) a.filt = *filt;
     else memset(&a.filt, 0, sizeof a.filt);
-    // shapes measured on MI355X for cohorts of 1, 10 and 16 streams:
-    //  - the logits head (51866 rows): one row per lane, 10 streams a block
-    //    (VALU-bound: ~1 FMA per weight element per stream), 2 blocks per CU,
-    //    weights through the batch pipeline;
+    // shapes measured on MI355X for cohorts of 1, 10 and 16 streams (many rows
+    // took fw_launch_gemm16x above):
+    //  - the logits head (51866 rows): one row per lane, weights through the
+    //    batch pipeline;
     //  - d x d (o, cross q/o): one stream per block, one row per lane (the
     //    most blocks; each re-reads the 3.3 MB matrix from L2 or the MALL);
     //  - q/k/v, fc1, fc2: 2 streams a block, 2 rows per lane; fc1 (N >= 4K)
