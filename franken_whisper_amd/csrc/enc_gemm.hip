@@ -448,8 +448,12 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
 //
 // The per-tile row scales sx, column scales sw and bias are staged into LDS
 // with the tile's first stage (SCL 256-byte loads per wave, the same number
-// for every wave so the counts above stay uniform; a tile's scales sit in the
-// LDS half of its parity).
+// for every wave so the counts above stay uniform), into one of SB = 4 slots by
+// the tile's number.  A stage is requested NS - 1 steps ahead and a step's
+// requests are not ordered against another wave's epilogue of the step before,
+// so tile t + SB may start to load from step (t + 1) n + 1 on at the earliest
+// (n steps a tile): (SB - 1) n >= NS.  With two slots that held from K = 64 NS
+// on, and a tile of K = 128 took the scales of the tile two further on.
 //
 // What bounds it: a 256 x 256 stage takes 1,550-1,750 cycles for 1,060 of MFMAs
 // (the stage barrier with both waves of a SIMD at it, LDS at three quarters of
@@ -465,18 +469,21 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
 // `wrows` > 0 (the QKV epilogue) M tiles never straddle a window of wrows rows:
 // each window is tiled on its own, so every tile's rows share one window and
 // start at a multiple of BM within it.
+#define PI8_MIN_K 128
 template <int EPI, int BM, int BN, int WGM, int WGN, int NS>
 __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_pi8(FwGemm g, int ntm, int ntn, int ntw) {
     constexpr int NW = WGM * WGN, WM = BM / WGM, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
     constexpr int STAGE = (BM + BN) * 64, LPW = STAGE / 1024 / NW;
     constexpr int SCL = (BM + 2 * BN + 64 * NW - 1) / (64 * NW); // scale loads per wave per tile
-    constexpr int SCLN = SCL * NW * 64;                           // floats per parity
+    constexpr int SCLN = SCL * NW * 64;                           // floats per slot
+    constexpr int SB = 4;                                         // slots
+    static_assert((SB - 1) * (PI8_MIN_K / 64) >= NS, "a slot is free before its next tile's scales arrive");
     constexpr bool QKV = EPI == FW_EPI_QKV;
     // wave-private LDS slab: QKV turns 32 x 32 f32 tiles (rows of 40), the
     // index epilogue sends 32 x WN u16 tiles out as whole rows
     constexpr int SLABB = QKV ? 32 * 40 * 4 : (EPI == FW_EPI_F16IDX ? 32 * WN * 2 : 0); // bytes per wave
     static_assert(STAGE % (1024 * NW) == 0, "stage loads must split evenly over waves");
-    __shared__ __align__(1024) unsigned char lds[NS * STAGE + 2 * SCLN * 4 + NW * SLABB];
+    __shared__ __align__(1024) unsigned char lds[NS * STAGE + SB * SCLN * 4 + NW * SLABB];
     float *scl = (float *)(lds + NS * STAGE);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
@@ -545,7 +552,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_pi8(FwGemm g, int nt
     // after a stage's last load: the scales of a new tile, the next stage
     auto advance = [&]() __attribute__((always_inline)) {
         if (it_step == 0) {
-            float *sd = scl + (it_tile & 1) * SCLN + wave * 64;
+            float *sd = scl + (it_tile % SB) * SCLN + wave * 64;
 #pragma unroll
             for (int e = 0; e < SCL; e++)
                 __builtin_amdgcn_global_load_lds((const void *)ssrc[e],
@@ -643,14 +650,14 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_pi8(FwGemm g, int nt
         // id, so per-element addresses are not hoisted out of the tile loop
         int ln = lane;
         asm volatile("" : "+v"(ln));
-        const float *ssx = scl + (tile & 1) * SCLN, *ssw = ssx + BM, *sbi = ssw + BN;
+        const float *ssx = scl + (tile % SB) * SCLN, *ssw = ssx + BM, *sbi = ssw + BN;
         // A 32 x WN u16 tile (accumulator layout: element r of lane l is row
         // (r/4)*8 + (l/32)*4 + r%4, column j*32 + l%32), put into this wave's
         // slab one 32-column tile j at a time, then flushed to rows dst + row*ld,
         // row < vrows, as 16-byte runs of whole rows (WN/8 lanes per row).  The
         // slab is private to the wave and a wave's LDS accesses run in order:
         // only the compiler must not reorder them.
-        uint16_t *const sl = (uint16_t *)(lds + NS * STAGE + 2 * SCLN * 4 + wave * SLABB);
+        uint16_t *const sl = (uint16_t *)(lds + NS * STAGE + SB * SCLN * 4 + wave * SLABB);
         auto slab_put = [&](int j, const uint16_t (&u)[16]) {
             asm volatile("" ::: "memory");
 #pragma unroll
@@ -788,7 +795,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_pi8(FwGemm g, int nt
                     }
                 }
         } else if constexpr (QKV) {
-            float *slab = (float *)(lds + NS * STAGE + 2 * SCLN * 4 + wave * SLABB);
+            float *slab = (float *)(lds + NS * STAGE + SB * SCLN * 4 + wave * SLABB);
             const int wnd = m0 / g.T, tb0 = m0 - wnd * g.T;
 #pragma unroll
             for (int i = 0; i < TM; i++)
@@ -955,7 +962,7 @@ bool fw_launch_gemm(hipStream_t st, int kind, const FwGemm &g0) {
         pi8 = e ? atoi(e) : 1;
     }
     if (kind == FW_KIND_F16S) return fw_launch_gemm_f16(st, g0, ncu);
-    if (pi8 && g.K % 64 == 0 &&
+    if (pi8 && g.K % 64 == 0 && g.K >= PI8_MIN_K &&
         (g.epi != FW_EPI_QKV || (g.T > 0 && g.M % g.T == 0))) {
         switch (g.epi) {
         case FW_EPI_F32: launch_pi8_tiles<FW_EPI_F32>(st, g, ncu); return true;

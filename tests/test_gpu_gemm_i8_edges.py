@@ -81,3 +81,54 @@ def test_fc1_index(pair, M):
     np.testing.assert_array_equal(gi[inside], y[inside].astype(np.float16).view(np.uint16))
     assert np.all(gi[~inside] == 0xFFFF)
     assert_bitexact(side.download()[~inside], y[~inside], "fc1 side values")
+
+
+# Width 128: a tile of K = 128 has two steps, fewer than the stages in flight, and
+# with more tiles than blocks a block's next tiles load their scales while it is
+# still at the last ones'.  Row counts for which a CU (256 of them) takes two and
+# three tiles.
+NARROW = synth.Config("i8-narrow", 51864, 1500, 128, 2, 1, 64, 128, 2, 1, 16)
+
+
+@pytest.fixture(scope="module")
+def narrow():
+    ctx = native.Context(0)
+    m = synth.Model(NARROW, seed=9, decoder=False)
+    e = native.Encoder(ctx, m, abi.ENC_INT8)
+    yield ctx, e, O.Encoder(m, abi.ENC_INT8)
+    e.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("M,which", [(66000, 0), (66000, 3), (33000, 4), (66000, 4), (66000, 5)])
+def test_narrow_rows(narrow, M, which):
+    ctx, e, oenc = narrow
+    d = NARROW.n_audio_state
+    inp, out = (4 * d if which == 5 else d), (4 * d if which == 4 else d)
+    rng = np.random.default_rng(M + which)
+    x = (rng.standard_normal((M, inp)) * rng.uniform(0.1, 3.0, (M, 1))).astype(np.float32)  # a scale of its own for every row
+    acc, y = ctx.empty((M, out), np.int32), ctx.empty((M, out), np.float32)
+    print("rows", M, "gemm", which, flush=True)
+    e.gemm_i8(0, which, ctx.array(x), acc, y)
+    want_acc, want_y = oenc.gemm(0, which, x)
+    np.testing.assert_array_equal(acc.download(), want_acc)
+    assert_bitexact(y.download(), want_y, f"rows {M} gemm {which}")
+
+
+@pytest.mark.parametrize("exact", [False, True], ids=["fast", "exact"])
+def test_narrow_windows(narrow, exact):
+    """44 and 64 windows through every epilogue of the forward (q/k/v split or
+    f32 rows, residual, index form): window for window the bits of a call with
+    that window alone."""
+    ctx, e, _ = narrow
+    e.set_exact(exact)
+    for n in (44,) if exact else (44, 64):
+        x = synth.mel_input(n, n, 3000, NARROW.n_mels) * np.float32(0.5)
+        out = ctx.empty((n, 1500, 128), np.float32)
+        print("windows", n, "exact", exact, flush=True)
+        e.forward_time_major(ctx.array(np.ascontiguousarray(x)), n, 3000, out)
+        got, one = out.download(), ctx.empty((1, 1500, 128), np.float32)
+        for w in (0, n // 3, n - 2, n - 1):
+            e.forward_time_major(ctx.array(np.ascontiguousarray(x[w:w + 1])), 1, 3000, one)
+            assert_bitexact(got[w], one.download()[0], f"window {w} of {n}")
+    e.set_exact(False)
