@@ -423,7 +423,7 @@ void fw_launch_gemv16(hipStream_t st, const uint16_t *Wp, const float *bias, con
                       const fwhip_filter *filt, const int *initialp, unsigned long long *keys, int r, int sb_cap,
                       int grid_cap) {
     const int n_cu = g_n_cu();
-    if (r <= 0 && sb_cap <= 0 && grid_cap <= 0 && fw_gemm16x_ok(N, K, ns)) {
+    if (r <= 0 && sb_cap <= 0 && grid_cap <= 0 && fw_gemm16x_ok(N, K, ns, keys != nullptr)) {
         fw_launch_gemm16x(st, Wp, bias, x, y, N, K, ns, ldy, mode, gelu_tab, lnw, lnb, filt, initialp, keys, n_cu);
         return;
     }

@@ -33,7 +33,7 @@ void fw_launch_gemv16(hipStream_t st, const uint16_t *Wp, const float *bias, con
                       const float *lnb = nullptr, const fwhip_filter *filt = nullptr, const int *initialp = nullptr,
                       unsigned long long *keys = nullptr, int r = 0, int sb_cap = 0, int grid_cap = 0);
 // The same on the matrix units, for many rows (dec_gemm16.hip).
-bool fw_gemm16x_ok(int N, int K, int ns);
+bool fw_gemm16x_ok(int N, int K, int ns, bool keys);
 void fw_launch_gemm16x(hipStream_t st, const uint16_t *Wp, const float *bias, const float *x, float *y, int N, int K,
                        int ns, int ldy, int mode, const float *gelu_tab, const float *lnw, const float *lnb,
                        const fwhip_filter *filt, const int *initialp, unsigned long long *keys, int n_cu);

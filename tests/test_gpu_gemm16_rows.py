@@ -56,3 +56,37 @@ def test_rows_match_single_rows(decs, d, S, n):
         assert_bitexact(got[s], one.download()[0], f"stream {s}")
         assert a[0] == am[s]
         ref.close()
+
+
+@pytest.mark.parametrize("V", [4096, 8192, 16383, 16384])
+@pytest.mark.parametrize("d,S", [(128, 10), (384, 16)])
+def test_small_vocabulary_argmax(d, S, V):
+    """A logits head of fewer than 16,384 rows: the cohort's argmax keys are
+    written at every step (the maximum moves from step to step), the tokens and
+    logits are those of one stream at a time."""
+    ctx = native.Context(0)
+    cfg = synth.Config(f"vocab-{V}-{d}", V, T, d, d // 64, 1, 448, d, d // 64, 1, 16)
+    m = synth.Model(cfg, seed=3, encoder=False)
+    dec = native.Decoder(ctx, m, abi.DEC_F16)
+    states = synth.encoder_states(7, S, T, d)
+    tokens = np.random.default_rng(V).integers(0, V, (S, 6)).astype(np.int32)
+    print("width", d, "streams", S, "vocabulary", V, flush=True)
+    st, out, one = dec.state(S, T), ctx.empty((S, V), np.float32), ctx.empty((1, V), np.float32)
+    st.set_cross(ctx.array(states))
+    cuts = [(0, 3), (3, 4), (4, 5), (5, 6)]  # a prompt, then single positions
+    got = []
+    for a, b in cuts:
+        am = st.step(tokens[:, a:b], out)
+        got.append((am, out.download()))
+        np.testing.assert_array_equal(am, got[-1][1].argmax(1))
+    assert len({tuple(am) for am, _ in got}) == len(cuts)
+    st.close()
+    for s in (0, S - 1):
+        ref = dec.state(1, T)
+        ref.set_cross(ctx.array(np.ascontiguousarray(states[s:s + 1])))
+        for (a, b), (am, logits) in zip(cuts, got):
+            assert ref.step(tokens[s:s + 1, a:b], one)[0] == am[s]
+            assert_bitexact(logits[s], one.download()[0], f"stream {s} positions {a}..{b}")
+        ref.close()
+    dec.close()
+    ctx.close()
