@@ -1255,8 +1255,10 @@ static double dec_step_bytes(const fwhip_dstate *st, int tk) {
 // argmax -> step.  Sampled tokens, the position and the step count live on the
 // device; each step after the first replays one captured graph; the host polls
 // for end-of-text every few steps, so steps stream without a per-token sync.
-// The pinned poll buffer of a state, at least n int32 (a poll copies a few
-// hundred bytes; pageable copies cost ~100 us of idle GPU each).
+// The pinned buffer of a state for what its decode loops copy to the host, at
+// least n int32 (a poll copies a few hundred bytes; pageable copies cost ~100 us
+// of idle GPU each, and the copy is then the stream's own work, complete when
+// the stream is).
 static int32_t *poll_buffer(fwhip_dstate *st, int n) {
     if (st->poll_cap < n) {
         if (st->poll_host) {
@@ -1300,12 +1302,11 @@ extern "C" fwhip_status fwhip_decode_greedy(fwhip_dstate *st, const int32_t *pro
     // first sampled token: from the prefill's logits
     fw_launch_argmax_finish(c->stream, st->keys, st->nkeys, S, st->tok, st->hist, st->hist_cap, st->pos, st->initial,
                             st->stepc, 1, st->am_cnt);
-    std::vector<int32_t> hist((size_t)S * n_max, -1);
     int steps = 1;
     const int poll = 8;
     // each poll copies the history's newest `poll` columns into pinned memory
     // and keeps which streams have produced end-of-text so far
-    int32_t *ph = poll_buffer(st, S * poll);
+    int32_t *ph = poll_buffer(st, S * (n_max > poll ? n_max : poll));
     if (!ph) return fw_fail(FWHIP_ERR_GENERIC, "pinned poll buffer");
     std::vector<uint8_t> done(S, 0);
     int polled = 0; // history columns already examined
@@ -1341,19 +1342,19 @@ extern "C" fwhip_status fwhip_decode_greedy(fwhip_dstate *st, const int32_t *pro
             if (all) break;
         }
     }
-    HIP_TRY(hipMemcpy2DAsync(hist.data(), sizeof(int32_t) * n_max, st->hist, sizeof(int32_t) * st->hist_cap,
+    HIP_TRY(hipMemcpy2DAsync(ph, sizeof(int32_t) * n_max, st->hist, sizeof(int32_t) * st->hist_cap,
                              sizeof(int32_t) * steps, S, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     HIP_TRY(hipGetLastError());
     for (int s = 0; s < S; s++) {
         int n = steps;
         for (int k = 0; k < steps; k++)
-            if (hist[(size_t)s * n_max + k] == filter->eot) {
+            if (ph[(size_t)s * n_max + k] == filter->eot) {
                 n = k + 1;
                 break;
             }
         out_len[s] = n;
-        for (int k = 0; k < n_max; k++) out_tokens[(size_t)s * n_max + k] = k < n ? hist[(size_t)s * n_max + k] : 0;
+        for (int k = 0; k < n_max; k++) out_tokens[(size_t)s * n_max + k] = k < n ? ph[(size_t)s * n_max + k] : 0;
     }
     st->len += n_prompt + steps - 1;
     return FWHIP_OK;
@@ -1500,7 +1501,10 @@ extern "C" fwhip_status fwhip_decode_window(fwhip_dstate *st, const int32_t *pro
                          st->w_forced, st->w_scratch, st->tok, st->pos, st->w_ndone, st->w_part, st->w_cnt, S);
     int steps = 1;
     const int poll = 8;
-    int32_t *pnd = poll_buffer(st, 1); // the done count, copied to pinned memory
+    // pinned: the done count of a poll; at the end the loop states, tokens,
+    // log-probabilities and no-speech rows
+    const size_t n_ws = (sizeof(FwWinStream) * S + 3) / 4, n_row = (size_t)S * n_max;
+    int32_t *pnd = poll_buffer(st, (int)(n_ws + 2 * n_row + S));
     if (!pnd) return fw_fail(FWHIP_ERR_GENERIC, "pinned poll buffer");
     bool use_graph = n_max > 1 && win_capture(st, cfg);
     for (int i = 1; i < n_max; i++) {
@@ -1527,27 +1531,28 @@ extern "C" fwhip_status fwhip_decode_window(fwhip_dstate *st, const int32_t *pro
     }
     fw_launch_win_plogs(c->stream, st->w_rows, st->w_nsrow, cfg, st->w_ws, st->hist, st->hist_cap, st->w_forced,
                         st->w_plogs, st->w_nslp, S);
-    std::vector<int32_t> hist((size_t)S * n_max);
-    std::vector<float> nslp(S);
-    HIP_TRY(hipMemcpyAsync(ws.data(), st->w_ws, sizeof(FwWinStream) * S, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpy2DAsync(hist.data(), sizeof(int32_t) * n_max, st->hist, sizeof(int32_t) * st->hist_cap,
+    const FwWinStream *fin = (const FwWinStream *)pnd;
+    int32_t *hist = pnd + n_ws;
+    float *plogs = (float *)(hist + n_row), *nslp = plogs + n_row;
+    HIP_TRY(hipMemcpyAsync(pnd, st->w_ws, sizeof(FwWinStream) * S, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipMemcpy2DAsync(hist, sizeof(int32_t) * n_max, st->hist, sizeof(int32_t) * st->hist_cap,
                              sizeof(int32_t) * n_max, S, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(out_plogs, st->w_plogs, sizeof(float) * S * n_max, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(nslp.data(), st->w_nslp, sizeof(float) * S, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipMemcpyAsync(plogs, st->w_plogs, sizeof(float) * S * n_max, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipMemcpyAsync(nslp, st->w_nslp, sizeof(float) * S, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     HIP_TRY(hipGetLastError());
     for (int s = 0; s < S; s++) {
-        const int n = ws[s].n_dec;
+        const int n = fin[s].n_dec;
         fwhip_window_stream &o = streams[s];
         o.n_tokens = n;
-        o.result_len = ws[s].result_len;
-        o.has_ts = ws[s].has_ts;
-        o.seek_delta_cs = ws[s].seek_delta_cs;
-        o.n_exact = ws[s].n_exact;
+        o.result_len = fin[s].result_len;
+        o.has_ts = fin[s].has_ts;
+        o.seek_delta_cs = fin[s].seek_delta_cs;
+        o.n_exact = fin[s].n_exact;
         o.no_speech_logprob = nslp[s];
         for (int k = 0; k < n_max; k++) {
             out_tokens[(size_t)s * n_max + k] = k < n ? hist[(size_t)s * n_max + k] : 0;
-            if (k >= n) out_plogs[(size_t)s * n_max + k] = 0.0f;
+            out_plogs[(size_t)s * n_max + k] = k < n ? plogs[(size_t)s * n_max + k] : 0.0f;
         }
     }
     st->len += n_prompt + steps - 1;
