@@ -263,7 +263,21 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_f16(FwGemm g, int nt
         const int wnd = m0 / g.T, tb0 = m0 - wnd * g.T;
         uint32_t of = 0;
 #pragma unroll
-        for (int i = 0; i < TM; i++)
+        for (int i = 0; i < TM; i++) {
+            // XKV: window and position of this lane's K row (lane / 2) and of the first
+            // row of its V^T runs
+            int kw = 0, kt = 0, vw[4], vt[4];
+            if constexpr (EPI == FW_EPI_XKV) {
+                const int rb = m0 + rw0 + i * 32;
+                kw = (rb + (lane >> 1)) / g.T;
+                kt = rb + (lane >> 1) - kw * g.T;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int row = rb + q * 8 + (lane >> 5) * 4;
+                    vw[q] = row / g.T;
+                    vt[q] = row - vw[q] * g.T;
+                }
+            }
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 const int c0 = col0 + j * 32, t0 = tb0 + rw0 + i * 32, vrows = mrows - (rw0 + i * 32);
@@ -279,7 +293,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_f16(FwGemm g, int nt
                     // column c0 + c = (l * 2 + kv) * d + h * 64 + dd: the 32 columns share l, kv and h
                     const int d = g.ldc, l = c0 / (2 * d), rc = c0 - l * 2 * d, kv = rc >= d ? 1 : 0, cc = rc - kv * d;
                     const int h = cc >> 6, dd0 = cc & 63;
-                    const size_t lh = ((size_t)wnd * g.L + l) * g.H + h;
+                    auto lh = [&](int w) { return ((size_t)w * g.L + l) * g.H + h; };
                     if (kv == 0) {
                         // K [T, 64] rows through the slab: 16 dims (32 bytes) per lane
                         asm volatile("" ::: "memory");
@@ -297,30 +311,41 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_f16(FwGemm g, int nt
 #pragma unroll
                             for (int q = 0; q < 8; q++)
                                 p[q] = fw_f2h(w4[q >> 1][(q & 1) * 2]) | ((uint32_t)fw_f2h(w4[q >> 1][(q & 1) * 2 + 1]) << 16);
-                            uint4 *o = (uint4 *)(g.o16[0] + (lh * g.T + t0 + row) * 64 + dd0 + half * 16);
+                            uint4 *o = (uint4 *)(g.o16[0] + (lh(kw) * g.T + kt) * 64 + dd0 + half * 16);
                             o[0] = make_uint4(p[0], p[1], p[2], p[3]);
                             o[1] = make_uint4(p[4], p[5], p[6], p[7]);
                         }
                     } else {
-                        // V^T [64, T]: a lane's runs of 4 keys
-                        uint16_t *o = g.o16[1] + (lh * 64 + dd0 + (ln & 31)) * g.T + t0;
+                        // V^T [64, T]: a lane's runs of 4 keys (with T % 4 == 0 all in one window)
 #pragma unroll
                         for (int q = 0; q < 4; q++) {
                             const int tr = q * 8 + (ln >> 5) * 4;
                             uint16_t u[4];
 #pragma unroll
                             for (int e = 0; e < 4; e++) u[e] = fw_f2h(acc[i][j][q * 4 + e] + bias[j]);
-                            if ((g.T & 3) == 0 && tr + 4 <= vrows) {
-                                *(uint2 *)(o + tr) = make_uint2(u[0] | ((uint32_t)u[1] << 16), u[2] | ((uint32_t)u[3] << 16));
+                            auto at = [&](int w, int t) {
+                                return g.o16[1] + (lh(w) * 64 + dd0 + (ln & 31)) * g.T + t;
+                            };
+                            if ((g.T & 3) == 0) {
+                                if (tr < vrows)
+                                    *(uint2 *)at(vw[q], vt[q]) =
+                                        make_uint2(u[0] | ((uint32_t)u[1] << 16), u[2] | ((uint32_t)u[3] << 16));
                             } else {
+                                int w = vw[q], t = vt[q];
 #pragma unroll
-                                for (int e = 0; e < 4; e++)
-                                    if (tr + e < vrows) o[tr + e] = u[e];
+                                for (int e = 0; e < 4; e++) {
+                                    if (tr + e < vrows) *at(w, t) = u[e];
+                                    if (++t == g.T) {
+                                        t = 0;
+                                        w++;
+                                    }
+                                }
                             }
                         }
                     }
                 }
             }
+        }
         if (of && g.ovf) *g.ovf = 1;
     } else if constexpr (C::GELU) {
         const uint16_t *tab = (const uint16_t *)lds;
@@ -426,7 +451,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_f16(FwGemm g, int nt
 template <int EPI, bool FL, int BM, int BN, int WGM, int WGN>
 static void launch_f16(hipStream_t st, const FwGemm &g) {
     int ntw = 0, ntm;
-    if (EPI == FW_EPI_QKV || EPI == FW_EPI_XKV) {
+    if (EPI == FW_EPI_QKV) {
         ntw = (g.T + BM - 1) / BM;
         ntm = (g.M / g.T) * ntw;
     } else {
@@ -439,7 +464,11 @@ static void launch_f16(hipStream_t st, const FwGemm &g) {
 
 template <int EPI, bool FL>
 static void pick_f16(hipStream_t st, const FwGemm &g, int ncu) {
-    constexpr bool win = EPI == FW_EPI_QKV || EPI == FW_EPI_XKV;
+    // q/k/v tiles stop at a window's end (V^T runs of 8 keys); the cross K/V's run
+    // over the windows: at 130 frames of 16 streams a window with tiles of its own is
+    // 2 of 128 rows for 130 (set_cross + one step 813 -> 764 us, 10 streams of 260
+    // frames 676 -> 607, 16 of 400 1,014 -> 957; from 1,500 frames on the same).
+    constexpr bool win = EPI == FW_EPI_QKV;
     constexpr bool gelu = EPI == FW_EPI_GELU_SPLIT || EPI == FW_EPI_CONV2;
     // Rounds of the CUs times a round's time relative to 256 x 256 tiles, one
     // block to a CU (measured, 8 windows: both planes 82 us for a round of 256 x

@@ -38,3 +38,34 @@ def test_cross_lengths(pair, T):
     st.close()
     for s in range(2):
         assert_bitexact(got[s], odec.state(states[s]).step(tokens[s]), f"stream {s}")
+
+
+@pytest.mark.parametrize("S,T", [(40, 1), (40, 2), (33, 3), (40, 4), (9, 31), (5, 33), (7, 50), (16, 66), (3, 127), (3, 130),
+                                 (5, 257), (7, 300), (2, 319), (40, 320)])
+def test_cross_kv_of_a_cohort(S, T):
+    """The fast cross K/V GEMM's tiles run over the streams' borders: every
+    stream's K and V^T are the bits that it gets alone, and within f16 rounding
+    of the strict ones (two f16 spacings of the largest value cover the f16
+    pair's 2^-22 and a rounding to the other neighbour)."""
+    ctx = native.Context(0)
+    cfg = synth.Config("cross-cohort", 51864, 320, 384, 6, 1, 64, 384, 6, 2, 16)
+    dec = native.Decoder(ctx, synth.Model(cfg, seed=6, encoder=False), abi.DEC_F16)
+    states = synth.encoder_states(T, S, T, cfg.n_text_state)
+    print("streams", S, "frames", T, flush=True)
+    st, one = dec.state(S, T), dec.state(1, T)
+    st.set_cross(ctx.array(states))
+    for s in range(S):
+        for exact in (False, True) if s in (0, S - 1) else (False,):
+            dec.set_exact(exact)
+            one.set_cross(ctx.array(np.ascontiguousarray(states[s:s + 1])))
+            for what in (abi.DS_CROSS_K_F16, abi.DS_CROSS_VT_F16):
+                got, want = st.read(what, s), one.read(what, 0)
+                if not exact:
+                    np.testing.assert_array_equal(got, want, err_msg=f"stream {s} buffer {what}")
+                else:
+                    g, w = got.view(np.float16).astype(np.float32), want.view(np.float16).astype(np.float32)
+                    assert np.abs(g - w).max() <= 2 * np.spacing(np.abs(want.view(np.float16)).max())
+    st.close()
+    one.close()
+    dec.close()
+    ctx.close()
