@@ -315,6 +315,7 @@ struct fwhip_dstate {
     // batched prompt prefill (f16 arm): activation rows of a chunk of
     // pf_chunk(S) positions x S streams, allocated on first use
     std::vector<void *> pf_owned;
+    hipEvent_t pf_ev = nullptr; // a layer of a long chunk done (cancellation inside it)
     float *pf_x = nullptr, *pf_h = nullptr, *pf_qkv = nullptr, *pf_att = nullptr, *pf_y = nullptr, *pf_ff = nullptr;
     FwWinPart *w_part = nullptr; // [S][WIN_NB] partial results of the select blocks
     int *w_cnt = nullptr;        // [S] select blocks counted in (zero between launches)
@@ -662,6 +663,7 @@ extern "C" void fwhip_dstate_free(fwhip_dstate *st) {
     fw_free_all(st->pf_owned);
     fw_free_all(st->owned);
     if (st->poll_host) hipHostFree(st->poll_host);
+    if (st->pf_ev) hipEventDestroy(st->pf_ev);
     delete st;
 }
 
@@ -1003,6 +1005,10 @@ static void dec_logits_f16(fwhip_dstate *st, const float *x, float *h, const fwh
 // forward gives it (decoder.rs:1754-1906).
 // A chunk is 32 positions, more while its rows stay within 256: the GEMMs'
 // 16-row tiles then fill the chip (one stream's 227 rows: 8 chunks of 32 before).
+// A chunk of more than 32 positions polls for cancellation after every layer,
+// with the next one already queued, so a cancelled call waits for a layer or two
+// (0.8 ms each at 227 turbo rows, the time of a 32-position chunk) and the GPU
+// never for the host.
 static int pf_chunk(int S) { return S >= 8 ? 32 : 256 / S; }
 static bool prefill_batch_ok(const fwhip_dstate *st) {
     const fwhip_decoder *dd = st->dec;
@@ -1012,6 +1018,7 @@ static bool prefill_batch_ok(const fwhip_dstate *st) {
 }
 static fwhip_status prefill_buffers(fwhip_dstate *st) {
     if (st->pf_x) return FWHIP_OK;
+    if (!st->pf_ev) HIP_TRY(hipEventCreateWithFlags(&st->pf_ev, hipEventDisableTiming));
     const fwhip_decoder *dd = st->dec;
     const size_t R = (size_t)st->S * pf_chunk(st->S), d = dd->d;
     st->pf_x = (float *)fw_dalloc(st->pf_owned, sizeof(float) * R * d);
@@ -1053,6 +1060,17 @@ static fwhip_status dec_forward_chunk(fwhip_dstate *st, const int32_t *tok, int 
         fw_gemv16(s, l.co16, l.co_b, att, x, d, d, R, d, 1, gt);
         fw_gemv16_ln(s, l.fc1_16, l.fc1_b, x, h, l.mlp_ln_w, l.mlp_ln_b, ff, dff, d, R, dff, 2, gt, sq);
         fw_gemv16(s, l.fc2_16, l.fc2_b, ff, x, d, dff, R, d, 1, gt);
+        if (n_pos > 32) {
+            if (li > 0) {
+                HIP_TRY(hipEventSynchronize(st->pf_ev));
+                const fwhip_status r = check_cancel(c);
+                if (r != FWHIP_OK) {
+                    hipStreamSynchronize(s);
+                    return r;
+                }
+            }
+            HIP_TRY(hipEventRecord(st->pf_ev, s));
+        }
     }
     // the last position's rows of every stream
     if (want_logits) dec_logits_f16(st, x + (size_t)(n_pos - 1) * S * d, h, filt, timed);

@@ -2,6 +2,9 @@
 device logits (decode.rs:702-867, 1708-1790) on adversarial rows, and
 cancellation of decoder calls (checkpoint() between prompt rows and sampled
 tokens, decode.rs:3566)."""
+import threading
+import time
+
 import numpy as np
 import pytest
 
@@ -88,5 +91,50 @@ def test_decoder_cancel_then_resume(ctx, arm):
     assert st.len == 0
     st.step(np.tile(tk.sot_sequence(), (2, 1)))
     assert st.len == len(tk.sot_sequence())
+    st.close()
+    dec.close()
+
+
+def test_long_prompt_is_cancelled_inside(ctx):
+    """A prompt that goes through the layers as one chunk (227 positions of one
+    stream, 24 layers) is cancelled by a request that comes while the GPU works on
+    it, well after the host has queued it; the state keeps its length, and the
+    same prompt then gives the same logits."""
+    cfg = synth.Config("cancel", 51864, 1500, 768, 12, 1, 448, 768, 12, 24, 16)
+    dec = native.Decoder(ctx, synth.Model(cfg, seed=2, encoder=False), abi.DEC_F16)
+    st = dec.state(1, 1500)
+    st.set_cross(ctx.array(enc_states(3, 1, 1500, 768)))
+    tokens = np.random.default_rng(4).integers(0, cfg.n_vocab, (1, 227)).astype(np.int32)
+    out = ctx.empty((1, cfg.n_vocab), np.float32)
+    took = []
+    for _ in range(3):
+        st.reset()
+        t = time.perf_counter()
+        st.step(tokens, out)
+        took.append(time.perf_counter() - t)
+    want = out.download()
+    for part in (0.4, 0.6):
+        st.reset()
+        start = threading.Event()
+
+        def later():
+            start.wait()
+            t = time.perf_counter()
+            while time.perf_counter() - t < part * min(took):
+                pass
+            ctx.cancel()
+
+        th = threading.Thread(target=later)
+        th.start()
+        start.set()
+        t = time.perf_counter()
+        with pytest.raises(native.FwhipError) as e:
+            st.step(tokens, out)
+        print("uncancelled", min(took), "asked at", part, "returned after", time.perf_counter() - t, flush=True)
+        th.join()
+        assert e.value.code == abi.ERR_CANCELLED
+        assert st.len == 0
+    st.step(tokens, out)
+    np.testing.assert_array_equal(out.download(), want)
     st.close()
     dec.close()
