@@ -220,7 +220,7 @@ def test_encoder_cancel_then_resume(ctx):
 
 @pytest.mark.parametrize("precision", [abi.ENC_INT8, abi.ENC_F32], ids=["int8", "f32"])
 def test_attention_tiles_bit_identical_across_batch_sizes(ctx, precision):
-    """large-v3-turbo: one window (128-query tiles), four (256) and six (512)
+    """large-v3-turbo: one window (128-query tiles), four (512) and six (256)
     give window 0 the same encoder states bit for bit, in both plans."""
     cfg = synth.TURBO
     m = synth.Model(cfg, seed=11, decoder=False)

@@ -11,7 +11,13 @@ for the whole f32 plan.  With six fc1 values of about 300 a row's maximum is
 about 300 * 0.03 * sqrt(6) = 22 (weights ~0.03): an index step there is at most
 2^-11 * 10 * 0.03 / 22 = 7e-6 and a few together stay under 1e-4, while a lo
 plane that is skipped or stale (2^-12 of 300 per value) would show as 1e-4 ..
-6e-4."""
+6e-4.
+The conv stem by itself (a model whose layers add nothing): the error of the
+pairs and f32 sums alone, bound 2e-5 max-abs of LayerNorm outputs around 1: K =
+1152 products at 2^-22 each and their sums give 1e-6; a conv2 value below 10 at the
+neighbouring f16 index of the GELU is off by 2^-7 in a row whose spread is 400 at
+these inputs, 5e-6 of a maximum of 4.  Without conv1's lo plane the same outputs are
+off by 2e-4 (checked in the test, in 64 bits on the CPU)."""
 import copy
 
 import numpy as np
@@ -53,6 +59,62 @@ def encs():
     for e in made.values():
         e.close()
     ctx.close()
+
+
+@pytest.fixture(scope="module")
+def stems():
+    """Encoders whose layers leave the rows as conv2 wrote them, and the model."""
+    ctx = native.Context(0)
+    m = copy.copy(synth.Model(CFG, seed=5, decoder=False))
+    m.t = dict(m.t)
+    for i in range(CFG.n_audio_layer):
+        for name in ("attn.out", "mlp.2"):
+            for part in ("weight", "bias"):
+                key = f"encoder.blocks.{i}.{name}.{part}"
+                m.t[key] = np.zeros_like(m.t[key])
+    made = {p: native.Encoder(ctx, m, p) for p in (abi.ENC_F32, abi.ENC_INT8)}
+    yield ctx, m, made
+    for e in made.values():
+        e.close()
+    ctx.close()
+
+
+def _gelu(x):
+    t = x.astype(np.float32).astype(np.float16).astype(np.float64)
+    y = (0.5 * t * (1 + np.tanh(0.7978846 * t * (1 + 0.044715 * t * t)))).astype(np.float16).astype(np.float64)
+    return np.where(x <= -10, 0.0, np.where(x >= 10, x, y))
+
+
+def _stem64(m, x, lo):
+    """ln_post of the conv stem of one window x [frames, mels] in 64 bits; lo: conv1's
+    outputs as f32, else as their f16 hi halves.  Also how many of them are >= 10."""
+    d, t = CFG.n_audio_state, x.shape[0]
+    w1, w2 = (m.t[f"encoder.conv{i}.weight"].view(np.float16).astype(np.float64) for i in (1, 2))
+    pad = np.pad(x.astype(np.float64), ((1, 1), (0, 0)))
+    h = _gelu(sum(pad[k:k + t] @ w1[:, :, k].T for k in range(3)) + m.t["encoder.conv1.bias"])
+    big = int((h >= 10).sum())
+    h = h.astype(np.float32 if lo else np.float16).astype(np.float64)
+    pad = np.pad(h, ((1, 1), (0, 0)))
+    y = _gelu(sum(pad[k:k + t:2] @ w2[:, :, k].T for k in range(3)) + m.t["encoder.conv2.bias"])
+    y = y + m.t["encoder.positional_embedding"].reshape(-1, d)[:t // 2]
+    y = y - y.mean(1, keepdims=True)
+    return y / np.sqrt((y * y).mean(1, keepdims=True) + 1e-5), big
+
+
+@pytest.mark.parametrize("plan", [abi.ENC_F32, abi.ENC_INT8], ids=["f32", "int8"])
+@pytest.mark.parametrize("rows,n", [(5, 7), (65, 9), (129, 4), (300, 3), (511, 3), (640, 4)])
+def test_conv_lo_plane(stems, rows, n, plan):
+    """conv1 outputs >= 10 (their lo halves are not zero), windows that end inside
+    row tiles: every window against the stem in 64 bits."""
+    ctx, m, made = stems
+    x = synth.mel_input(rows, n, 2 * rows, CFG.n_mels) * np.float32(15000.0)
+    got = _forward(ctx, made[plan], x, rows)
+    for w in range(n):
+        want, big = _stem64(m, x[w], True)
+        err, lost = rel_maxabs(got[w], want.astype(np.float32)), rel_maxabs(_stem64(m, x[w], False)[0], want)
+        print("rows", rows, "window", w, "large", big, "error", err, "without lo", lost, flush=True)
+        assert big > rows * 2 * CFG.n_audio_state // 5 and lost > 5e-5
+        assert err < 2e-5
 
 
 def _forward(ctx, e, x, rows, exact=False):

@@ -1,7 +1,8 @@
-"""The int8 encoder GEMMs at the edges of their tiles (256 x 256, 256 x 128, 128 x
-128 and where the choice between them changes): the exact accumulators and
-every epilogue against the oracle bit for bit, the fused q/k/v split against the
-f16 pairs of the oracle's values."""
+"""The int8 encoder GEMMs at the edges of their tiles (256 x 256, 256 x 128 and
+128 x 128, the choice as on 256 CUs): the exact accumulators and the f32 rows
+against the oracle bit for bit, the fused q/k/v split against the f16 pairs of
+the oracle's values, fc1's index form; the residual epilogue through whole
+forwards, window for window the bits of a window alone."""
 import numpy as np
 import pytest
 
@@ -40,7 +41,9 @@ def test_gemm_rows(pair, M):
         assert_bitexact(y.download(), want_y, f"rows {M} gemm {which}")
 
 
-@pytest.mark.parametrize("B,T", [(1, 1), (3, 31), (2, 64), (1, 129), (5, 255), (2, 257), (1, 1500), (30, 300)])
+@pytest.mark.parametrize("B,T", [(1, 1), (3, 31), (2, 64), (1, 129), (5, 255), (2, 257), (1, 1500), (30, 300),
+                                 (10, 257), (14, 259), (8, 639),  # 256 x 128
+                                 (12, 513), (7, 1025), (9, 769), (16, 511)])  # 256 x 256
 def test_qkv_windows(pair, B, T):
     ctx, e, oenc = pair
     d, H, Tp = CFG.n_audio_state, CFG.n_audio_head, (T + 63) // 64 * 64
@@ -81,6 +84,21 @@ def test_fc1_index(pair, M):
     np.testing.assert_array_equal(gi[inside], y[inside].astype(np.float16).view(np.uint16))
     assert np.all(gi[~inside] == 0xFFFF)
     assert_bitexact(side.download()[~inside], y[~inside], "fc1 side values")
+
+
+@pytest.mark.parametrize("n,rows", [(5, 37), (3, 129), (14, 1499), (15, 1411)])
+def test_residual_windows(pair, n, rows):
+    """attn.out and fc2 add into the rows that they update: 128 x 128 tiles (few
+    rows), 256 x 128 (21,000), with a last tile of a few rows."""
+    ctx, e, _ = pair
+    x = synth.mel_input(n, n, 2 * rows, CFG.n_mels) * np.float32(0.5)
+    out, one = ctx.empty((n, rows, 384), np.float32), ctx.empty((1, rows, 384), np.float32)
+    print("windows", n, "rows", rows, flush=True)
+    e.forward_time_major(ctx.array(np.ascontiguousarray(x)), n, 2 * rows, out)
+    got = out.download()
+    for w in sorted({0, n // 2, n - 1}):
+        e.forward_time_major(ctx.array(np.ascontiguousarray(x[w:w + 1])), 1, 2 * rows, one)
+        assert_bitexact(got[w], one.download()[0], f"window {w} of {n}")
 
 
 # Width 128: a tile of K = 128 has two steps, fewer than the stages in flight, and
