@@ -7,16 +7,15 @@
 // (nn.rs:1660-1700, encoder.rs:2573-2580).  (The f16-pair GEMMs are in
 // enc_gemm_f16.hip.)
 //
-// Block = 256 threads as 2x2 waves; block tile BM x BN (128x128 by default;
-// 256x256 and 256x128 for sweeps);
-// each wave owns (BM/2) x (BN/2) as a grid of 32x32 MFMA tiles.  K advances
-// 64 bytes per stage; a stage is staged global ->
-// registers -> LDS (rows padded to 80 bytes: conflict-free 16-byte reads),
-// double buffered with one barrier per stage.  The epilogue is a template
-// parameter so its loops fully unroll and the accumulators stay in registers.
+// Two kernels, the same bits: k_gemm_pi8, persistent blocks over 256 x 256, 256 x
+// 128 or 128 x 128 tiles, which the encoder runs, and k_gemm_tile, a 128 x 128 tile
+// a block with its epilogue on its own, to check the first against
+// (FWHIP_GEMM_I8P=0).  In both, K advances 64 bytes per stage, global -> LDS
+// directly, and the epilogue is a template parameter so its loops unroll and
+// the accumulators stay in registers.
 //
 // Tile order: the hardware deals blocks round-robin to the 8 XCDs; block ids
-// are remapped so each XCD gets a contiguous run of tiles, walked in groups of
+// are mapped so each XCD gets a contiguous run of tiles, walked in groups of
 // 8 M-tiles (N outer), so an XCD's L2 holds the A rows of its group and one B
 // tile at a time.
 //
@@ -24,11 +23,8 @@
 // bytes; B lane l -> col l%32, same k block; accumulator r of lane l -> row
 // (r/4)*8 + (l/32)*4 + r%4, col l%32.
 #include <cstdlib>
-#include <cstring>
 
 #include "enc_gemm.h"
-
-#define GEMM_LDSR 80 // LDS row stride in bytes (64 data + 16 pad)
 
 __global__ void __launch_bounds__(256) k_split_f16(const float4 *x, size_t n4, uint2 *hi, uint2 *lo, int *ovf) {
     uint32_t of = 0;
@@ -53,6 +49,9 @@ void fw_launch_split_f16(hipStream_t st, const float *x, size_t n, uint16_t *hi,
     hipLaunchKernelGGL(k_split_f16, dim3((unsigned)g), dim3(256), 0, st, (const float4 *)x, n4, (uint2 *)hi,
                        (uint2 *)lo, ovf);
 }
+
+#define GT_BM 128 // k_gemm_tile's block tile
+#define GT_BN 128
 
 // Epilogue for the 4 consecutive rows row0..row0+3 of one column.
 template <int EPI>
@@ -222,105 +221,16 @@ __device__ __forceinline__ void gemm_epilogue(const FwGemm &g, v16i (&acc)[BM / 
         }
 }
 
-template <int EPI, int BM, int BN>
-__global__ void __launch_bounds__(256) k_gemm(FwGemm g, int ntm, int ntn) {
-    constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-    constexpr int ROWS = BM + BN; // LDS rows per stage
-    constexpr int STAGE = ROWS * GEMM_LDSR;
-    constexpr int CH = ROWS * 4 / 256; // 16-byte chunks per thread per stage
-    constexpr int CHA = BM / 64;  // chunks (per thread) that belong to A
-    __shared__ __align__(16) unsigned char lds[2 * STAGE];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-
-    // XCD-contiguous, M-grouped tile order
-    const int t = gemm_tile_order(g.map);
-    constexpr int GM = 8;
-    const int gsize = GM * ntn, grp = t / gsize, first_m = grp * GM;
-    const int gm = min(ntm - first_m, GM), rr = t - grp * gsize;
-    const int m0 = (first_m + rr % gm) * BM, n0 = (rr / gm) * BN;
-    const int nsteps = g.K / 64;
-
-    int4 stg[CH];
-    auto gload = [&](int s) {
-#pragma unroll
-        for (int q = 0; q < CH; q++) {
-            const int row = (tid >> 2) + q * 64, cc = tid & 3;
-            const size_t koff = (size_t)s * 64 + cc * 16;
-            if (q < CHA) {
-                const int gr = m0 + row;
-                const unsigned char *base = (const unsigned char *)g.A;
-                stg[q] = gr < g.M ? *(const int4 *)(base + (size_t)gr * g.lda + koff) : make_int4(0, 0, 0, 0);
-            } else {
-                const int gn = n0 + row - BM;
-                stg[q] = gn < g.N ? *(const int4 *)((const unsigned char *)g.B + (size_t)gn * g.ldb + koff)
-                                  : make_int4(0, 0, 0, 0);
-            }
-        }
-    };
-    auto lstore = [&](int buf) {
-        unsigned char *base = lds + buf * STAGE;
-#pragma unroll
-        for (int q = 0; q < CH; q++) {
-            const int row = (tid >> 2) + q * 64, cc = tid & 3;
-            *(int4 *)(base + row * GEMM_LDSR + cc * 16) = stg[q];
-        }
-    };
-
-    v16i acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0;
-
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    int buf = 0;
-    for (int s = 0; s < nsteps; s++) {
-        if (s + 1 < nsteps) gload(s + 1);
-        const unsigned char *tb = lds + buf * STAGE;
-#pragma unroll
-        for (int ks = 0; ks < 2; ks++) {
-            const int koff = ks * 32 + (lane >> 5) * 16;
-            v4i af[TM], bf[TN];
-#pragma unroll
-            for (int i = 0; i < TM; i++) {
-                const int row = wm * WM + i * 32 + (lane & 31);
-                af[i] = *(const v4i *)(tb + row * GEMM_LDSR + koff);
-            }
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const int row = wn * WN + j * 32 + (lane & 31);
-                bf[j] = *(const v4i *)(tb + (BM + row) * GEMM_LDSR + koff);
-            }
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int j = 0; j < TN; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], acc[i][j], 0, 0, 0);
-        }
-        if (s + 1 < nsteps) lstore(buf ^ 1);
-        __syncthreads();
-        buf ^= 1;
-    }
-
-    gemm_epilogue<EPI, BM, BN>(g, acc, lds, m0, n0);
-}
-
 // ---------------------------------------------------------------------------
-// Pipelined variant: operands go global -> LDS directly
+// One tile per block, 2x2 waves: operands go global -> LDS directly
 // (global_load_lds_dwordx4, no staging registers), NS stages in flight, one
 // barrier per stage.  LDS rows are 64 bytes with the 16-byte chunks of row r
 // XOR-swizzled by (r ^ r>>2) & 3, so the MFMA fragment reads are free of bank
 // conflicts.  Each wave loads ROWS/64 row groups of 16 rows per stage (one
 // instruction writes 16 rows x 64 bytes = 1 KB contiguous in LDS).
-
-
-template <int EPI, int BM, int BN, int NS>
-__global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
+template <int EPI>
+__global__ void __launch_bounds__(256) k_gemm_tile(FwGemm g, int ntm, int ntn) {
+    constexpr int BM = GT_BM, BN = GT_BN, NS = 3;
     constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
     constexpr int ROWS = BM + BN;
     constexpr int STAGE = ROWS * 64;
@@ -428,7 +338,7 @@ __global__ void __launch_bounds__(256) k_gemm2(FwGemm g, int ntm, int ntn) {
 }
 
 // ---------------------------------------------------------------------------
-// Persistent int8 GEMM.  One block per CU walks its share of the tile sequence
+// Persistent int8 GEMM.  A block (one or two to a CU) walks its share of the tile sequence
 // through a single flattened (tile, k-step) pipeline: the operand stages of the
 // next tile are already in flight while the current tile's epilogue runs, and
 // its stores drain to memory under the next tile's MFMAs (a one-tile-per-block
@@ -842,62 +752,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_pi8(FwGemm g, int nt
 }
 
 // ---------------------------------------------------------------------------
-// Tile choice: register-staged tiles (r256x256, r256x128, r128x128) and the
-// pipelined direct-to-LDS tiles (p256x256, p256x128, p128x128 with 4 stages,
-// or 2-3 stages: n2, n3).  FWHIP_GEMM_TILE=<name> forces one (tuning sweeps).
-static const char *kTileNames[9] = {"r256x256", "r256x128", "r128x128", "p256x256", "p256x128",
-                                    "p128x128", "p256x128n2", "p128x128n3", "p128x128n2"};
-
-static int forced_tile() {
-    static int forced = -2;
-    if (forced == -2) {
-        forced = -1;
-        const char *e = getenv("FWHIP_GEMM_TILE");
-        if (e)
-            for (int i = 0; i < 9; i++)
-                if (!strcmp(e, kTileNames[i])) forced = i;
-    }
-    return forced;
-}
-
-// Measured (large-v3-turbo int8 plan, 10 windows): p128x128 with 3 stages
-// (three blocks per CU, so one block's epilogue overlaps the others' MFMAs)
-// 885 TOP/s over the encoder's GEMMs, ahead of every other variant
-// (p128x128n2 816, p128x128 851, p256x128n2 722, p256x256 640).
-static int pick_tile(int M, int N, int ncu) {
-    int f = forced_tile();
-    if (f >= 0) return f;
-    (void)M;
-    (void)N;
-    (void)ncu;
-    return 7;
-}
-
-template <int EPI, int BM, int BN>
-static void launch_one(hipStream_t st, const FwGemm &g) {
-    int ntm = (g.M + BM - 1) / BM, ntn = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL((k_gemm<EPI, BM, BN>), dim3(ntm * ntn), dim3(256), 0, st, g, ntm, ntn);
-}
-
-template <int EPI, int BM, int BN, int NS>
-static void launch_pipe(hipStream_t st, const FwGemm &g) {
-    int ntm = (g.M + BM - 1) / BM, ntn = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL((k_gemm2<EPI, BM, BN, NS>), dim3(ntm * ntn), dim3(256), 0, st, g, ntm, ntn);
-}
-
 template <int EPI>
-static void launch_tiles(hipStream_t st, const FwGemm &g, int tile) {
-    switch (tile) {
-    case 0: launch_one<EPI, 256, 256>(st, g); break;
-    case 1: launch_one<EPI, 256, 128>(st, g); break;
-    case 2: launch_one<EPI, 128, 128>(st, g); break;
-    case 3: launch_pipe<EPI, 256, 256, 4>(st, g); break;
-    case 4: launch_pipe<EPI, 256, 128, 4>(st, g); break;
-    case 5: launch_pipe<EPI, 128, 128, 4>(st, g); break;
-    case 6: launch_pipe<EPI, 256, 128, 2>(st, g); break;
-    case 7: launch_pipe<EPI, 128, 128, 3>(st, g); break;
-    default: launch_pipe<EPI, 128, 128, 2>(st, g); break;
-    }
+static void launch_tile(hipStream_t st, const FwGemm &g) {
+    const int ntm = (g.M + GT_BM - 1) / GT_BM, ntn = (g.N + GT_BN - 1) / GT_BN;
+    hipLaunchKernelGGL(k_gemm_tile<EPI>, dim3(ntm * ntn), dim3(256), 0, st, g, ntm, ntn);
 }
 
 // Persistent int8 launch.  256x256 tiles (8 waves of 128x64) or 256x128 (8 of
@@ -964,7 +822,8 @@ bool fw_launch_gemm(hipStream_t st, int kind, const FwGemm &g0) {
         pi8 = e ? atoi(e) : 1;
     }
     if (kind == FW_KIND_F16S) return fw_launch_gemm_f16(st, g0, ncu);
-    if (pi8 && g.K % 64 == 0 && g.K >= PI8_MIN_K &&
+    if (g.K % 64) return false;
+    if (pi8 && g.K >= PI8_MIN_K &&
         (g.epi != FW_EPI_QKV || (g.T > 0 && g.M % g.T == 0))) {
         switch (g.epi) {
         case FW_EPI_F32: launch_pi8_tiles<FW_EPI_F32>(st, g, ncu); return true;
@@ -975,12 +834,11 @@ bool fw_launch_gemm(hipStream_t st, int kind, const FwGemm &g0) {
         default: break;
         }
     }
-    int tile = pick_tile(g.M, g.N, ncu);
     switch (g.epi) {
-    case FW_EPI_F32: launch_tiles<FW_EPI_F32>(st, g, tile); return true;
-    case FW_EPI_RESID: launch_tiles<FW_EPI_RESID>(st, g, tile); return true;
-    case FW_EPI_QKV: launch_tiles<FW_EPI_QKV>(st, g, tile); return true;
-    case FW_EPI_ACC32: launch_tiles<FW_EPI_ACC32>(st, g, tile); return true;
+    case FW_EPI_F32: launch_tile<FW_EPI_F32>(st, g); return true;
+    case FW_EPI_RESID: launch_tile<FW_EPI_RESID>(st, g); return true;
+    case FW_EPI_QKV: launch_tile<FW_EPI_QKV>(st, g); return true;
+    case FW_EPI_ACC32: launch_tile<FW_EPI_ACC32>(st, g); return true;
     default: return false;
     }
 }

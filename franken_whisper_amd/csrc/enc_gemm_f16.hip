@@ -235,7 +235,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_f16(FwGemm g, int nt
     float bias[TN];
 #pragma unroll
     for (int j = 0; j < TN; j++) bias[j] = g.bias ? g.bias[min(col0 + j * 32 + (lane & 31), g.N - 1)] : 0.0f;
-    if constexpr (EPI == FW_EPI_F32 || EPI == FW_EPI_RESID) {
+    if constexpr (EPI == FW_EPI_RESID) {
         // the residual values of the next 32x32 tile are requested before a tile's stores
         float cv[2][16];
         auto fetch = [&](int x) {
@@ -244,17 +244,16 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) k_gemm_f16(FwGemm g, int nt
             for (int r = 0; r < 16; r++)
                 cv[x & 1][r] = g.C[(size_t)(m0 + min(rowl(x / TN, r), mrows - 1)) * g.ldc + col];
         };
-        if constexpr (EPI == FW_EPI_RESID) fetch(0);
+        fetch(0);
 #pragma unroll
         for (int x = 0; x < TM * TN; x++) {
             const int i = x / TN, j = x % TN, col = col0 + j * 32 + (lane & 31);
-            if constexpr (EPI == FW_EPI_RESID)
-                if (x + 1 < TM * TN) fetch(x + 1);
+            if (x + 1 < TM * TN) fetch(x + 1);
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 float v = acc[i][j][r];
                 if (g.bias) v = v + bias[j];
-                if constexpr (EPI == FW_EPI_RESID) v = cv[x & 1][r] + v;
+                v = cv[x & 1][r] + v;
                 if (rowl(i, r) < mrows && col < g.N) g.C[(size_t)(m0 + rowl(i, r)) * g.ldc + col] = v;
             }
         }
