@@ -46,7 +46,8 @@ def _classes():
         abi.K_DEC_CROSS: ("decoder cross K/V precompute (k_gemm_f16 f16 pairs, all layers)", "mfma", "f16", None),
         abi.K_DEC_STEP: ("decoder step (graph replay of one sampled step: weights + cross K/V + KV cache)",
                          "hbm", None, "dec_step"),
-        abi.K_DEC_LOGITS: ("decoder logits GEMV of the prompt row (k_gemv_i8m)", "hbm", None, None),
+        abi.K_DEC_LOGITS: ("decoder logits head of the prompt row (k_gemm16x from 6 streams on, k_gemv16; int8 arm: "
+                           "k_gemv_i8m)", "hbm", None, None),
     }
 
 

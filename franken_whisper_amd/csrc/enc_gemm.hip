@@ -366,12 +366,14 @@ __global__ void __launch_bounds__(256) k_gemm_tile(FwGemm g, int ntm, int ntn) {
 // on, and a tile of K = 128 took the scales of the tile two further on.
 //
 // What bounds it: a 256 x 256 stage takes 1,550-1,750 cycles for 1,060 of MFMAs
-// (the stage barrier with both waves of a SIMD at it, LDS at three quarters of
-// its rate), a tile's epilogue 15,000-18,000 against 35,000 for its 20 stages at K
-// 1280 (conversion of the accumulators, store instructions), the clock falls to
-// 1.6-1.9 GHz under it.  With the loads and fragment reads between the MFMAs
-// instead of after the barrier (10 windows): q/k/v 146 -> 127 us, attn.out 66 ->
-// 56, fc1 150 -> 146, fc2 165 -> 155.
+// (the stage barrier with both waves of a SIMD at it; the fragments, 96 KB a stage
+// and CU, would be three quarters of the LDS rate if the MFMAs ran back to back and
+// are half of it as it is), a tile's epilogue 15,000-18,000 against 35,000 for its
+// 20 stages at K 1280 (conversion of the accumulators, store instructions), the
+// clock falls to 1.6-1.9 GHz under it.  With the loads and fragment reads between
+// the MFMAs instead of after the barrier (10 windows): a kernel back to back with
+// itself q/k/v 146 -> 127 us, attn.out 66 -> 56, fc1 150 -> 146, fc2 165 -> 155; in
+// the encoder's trace 144 -> 140, 72 -> 68, 158 -> 157, 178 both.
 //
 // Tile sequence: XCD x (blocks x, x+8, ...) owns a contiguous range of the
 // GM=8-grouped tile order, walked by its blocks in lockstep, so the tiles in

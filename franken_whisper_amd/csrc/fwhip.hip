@@ -1276,7 +1276,9 @@ static double dec_step_bytes(const fwhip_dstate *st, int tk) {
 // The pinned buffer of a state for what its decode loops copy to the host, at
 // least n int32 (a poll copies a few hundred bytes; pageable copies cost ~100 us
 // of idle GPU each, and the copy is then the stream's own work, complete when
-// the stream is).
+// the stream is: under rocprofv3 a strided copy into a pageable vector had written
+// nothing when hipStreamSynchronize returned, and every token read as the
+// vector's initial -1).
 static int32_t *poll_buffer(fwhip_dstate *st, int n) {
     if (st->poll_cap < n) {
         if (st->poll_host) {
