@@ -260,8 +260,11 @@ void gx_go(hipStream_t st, int grid_cap, const uint16_t *Wp, const float *bias, 
 // outputs fill the chip (10 rows: fc1 11.9 -> 10.9 us; 16: q/k/v 12.7 -> 11.9, fc1
 // 15.1 -> 12.1; 32: cross q 13.9 -> 11.9, q/k/v 20.8 -> 12.4, fc1 28 -> 23; 320:
 // d x d 68 -> 43, fc1 254 -> 152).  Rows longer than 1,280 (fc2) gained nothing.
-// Argmax keys (a logits head) are formed in the eight-lane form alone: a
-// vocabulary below 16,384 stays with the vector kernel.
+// The other widths were not fitted, but they gain by the same thresholds: whole
+// decodes of 6-16 streams at widths 384, 512, 768 and 1,024 1.01-1.19x, prompts of
+// 4-200 rows 1.07-2.7x, one to five streams unchanged.  Argmax keys (a logits
+// head) are formed in the eight-lane form alone: a vocabulary below 16,384 stays
+// with the vector kernel.
 bool fw_gemm16x_ok(int N, int K, int ns, bool keys) {
     const int lpr = fw_gemv16_lpr(N, K);
     if (K > GX_K || (lpr != 8 && lpr != 16) || K % (lpr == 8 ? 64 : 128) || (keys && lpr != 8)) return false;

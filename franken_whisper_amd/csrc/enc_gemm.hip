@@ -768,7 +768,10 @@ static void launch_tile(hipStream_t st, const FwGemm &g) {
 // The choice is the fewest rounds of the CUs, weighted by a round's time
 // relative to 256x256 (measured, K 1280, 10 windows: 27 us, 15 for 256x128, 16
 // for two 128x128 a CU, less where one a CU suffices: one and two windows' fc2
-// 47 -> 39 us).
+// 47 -> 39 us).  Used at every width: with it, and the attention and stem that
+// came beside it, whole int8 encoder calls of widths 384-1,280 over 1-16 windows of
+// 50-1,500 rows ran 1.10-1.37x faster than with the tile by the output's width
+// alone, none slower.
 template <int EPI, int BM, int BN, int WGM, int WGN, int NS>
 static void launch_pi8(hipStream_t st, const FwGemm &g, int ncu, int per_cu) {
     int ntw = 0, ntm;
